@@ -6,6 +6,19 @@
 #include <hip/hip_runtime_api.h>
 #include "fn2_kernel_args.h"
 
+namespace fn2
+{
+    // Density blocks of one face-count launch, passed by value, and the
+    // { quads, solid } entries its blocks write at most
+    // (fn2_face_blocks( n, gen ) per chunk, n <= kFaceJobs)
+    constexpr int kFaceJobs = 64;
+    constexpr int kFaceEntries = 2048;
+    struct FaceJobs
+    {
+        const float* density[kFaceJobs];
+    };
+}
+
 extern "C" {
 // one interpreter launch over args->total points
 int fn2_launch_generate( const fn2::GenArgs* args, int dimMask, int featMask, hipStream_t stream );
@@ -26,6 +39,9 @@ int fn2_launch_batch_init( int32_t* keys, int n, int slots, int stride, uint32_t
 int fn2_batch_block_threads( void );
 // device-side checks of the math helpers
 int fn2_launch_selftest_math( int op, const float* in, float* out, int n, hipStream_t stream );
-// faces of a bloxel mesh of a gen^3 density block
-int fn2_launch_bloxel_faces( const float* density, int gen, float iso, uint32_t* counts, hipStream_t stream );
+// faces of the bloxel meshes of n gen^3 density blocks (divS divides by
+// gen - 2): fn2_face_blocks( n, gen ) entries of { quads, solid } per block,
+// chunk after chunk, into `partials`
+int fn2_face_blocks( int n, int gen );
+int fn2_launch_bloxel_faces( const fn2::FaceJobs* jobs, int n, int gen, fn2::FastDiv divS, float iso, uint32_t* partials, hipStream_t stream );
 }

@@ -90,8 +90,7 @@ namespace
             // requests still in flight write into the buffers: let them finish
             for( Pending& p : inflight ) fn2ServeWait( engine, p.request, nullptr, nullptr );
             for( float* b : buffers ) if( b ) ( void )hipFree( b );
-            if( dCounts ) ( void )hipFree( dCounts );
-            if( hCounts ) ( void )hipHostFree( hCounts );
+            if( hFaces ) ( void )hipHostFree( hFaces );
             if( stream ) ( void )hipStreamDestroy( stream );
         }
 
@@ -102,8 +101,9 @@ namespace
             for( float*& b : buffers )
                 if( hipMalloc( (void**)&b, bytes ) != hipSuccess ) { ( void )hipGetLastError(); initError = "hipMalloc(chunk density)"; return false; }
             for( int i = maxInFlight - 1; i >= 0; i-- ) freeBuffers.push_back( i );
-            if( hipMalloc( (void**)&dCounts, sizeof( uint32_t ) * 2 * maxInFlight ) != hipSuccess ||
-                hipHostMalloc( (void**)&hCounts, sizeof( uint32_t ) * 2 * maxInFlight, hipHostMallocDefault ) != hipSuccess ||
+            const size_t launches = ( (size_t)maxInFlight + fn2::kFaceJobs - 1 ) / fn2::kFaceJobs;
+            divSize = fn2::MakeFastDiv( (uint32_t)size );
+            if( hipHostMalloc( (void**)&hFaces, launches * fn2::kFaceEntries * 2 * sizeof( uint32_t ), hipHostMallocDefault ) != hipSuccess ||
                 hipStreamCreateWithFlags( &stream, hipStreamNonBlocking ) != hipSuccess )
             {
                 ( void )hipGetLastError();
@@ -177,26 +177,34 @@ namespace
                 done.push_back( { *it, { mm[0], mm[1] } } );
                 it = inflight.erase( it );
             }
-            // consumer kernels for the chunks whose range straddles the iso surface
+            // consumer kernels for the chunks whose range straddles the iso
+            // surface, kFaceJobs chunks a launch
             std::vector<int> state( done.size() );
-            bool launched = false;
+            std::vector<size_t> surface;
             for( size_t i = 0; i < done.size(); i++ )
             {
                 const Done& d = done[i];
                 if( d.p.version != version ) continue;
                 state[i] = d.mm[0] > iso ? FN2_CHUNK_AIR : d.mm[1] < iso ? FN2_CHUNK_SOLID : FN2_CHUNK_SURFACE;
-                if( state[i] != FN2_CHUNK_SURFACE ) continue;
-                uint32_t* counts = dCounts + 2 * d.p.buffer;
-                if( !fn2::HipOk( hipMemsetAsync( counts, 0, 2 * sizeof( uint32_t ), stream ), "chunk counters" ) ||
-                    !fn2::HipOk( (hipError_t)fn2_launch_bloxel_faces( buffers[d.p.buffer], gen, iso, counts, stream ), "chunk faces" ) )
-                    return -1;
-                launched = true;
+                if( state[i] == FN2_CHUNK_SURFACE ) surface.push_back( i );
             }
-            if( launched )
+            std::vector<std::array<uint32_t, 2>> faces( done.size() );   // { quads, solid voxels }
+            for( size_t first = 0; first < surface.size(); first += fn2::kFaceJobs )
             {
-                if( !fn2::HipOk( hipMemcpyAsync( hCounts, dCounts, sizeof( uint32_t ) * 2 * maxInFlight, hipMemcpyDeviceToHost, stream ), "chunk counts" ) ||
-                    !fn2::HipOk( hipStreamSynchronize( stream ), "chunk consumer" ) )
-                    return -1;
+                const int jobs = (int)std::min<size_t>( fn2::kFaceJobs, surface.size() - first );
+                fn2::FaceJobs fj{};
+                for( int j = 0; j < jobs; j++ ) fj.density[j] = buffers[done[surface[first + j]].p.buffer];
+                if( !fn2::HipOk( (hipError_t)fn2_launch_bloxel_faces( &fj, jobs, gen, divSize, iso, FacesOf( first ), stream ), "chunk faces" ) ) return -1;
+            }
+            if( !surface.empty() && !fn2::HipOk( hipStreamSynchronize( stream ), "chunk consumer" ) ) return -1;
+            for( size_t first = 0; first < surface.size(); first += fn2::kFaceJobs )
+            {
+                const int jobs = (int)std::min<size_t>( fn2::kFaceJobs, surface.size() - first );
+                const int blocks = fn2_face_blocks( jobs, gen );
+                const uint32_t* e = FacesOf( first );
+                for( int j = 0; j < jobs; j++ )
+                    for( int b = 0; b < blocks; b++, e += 2 )
+                        for( int v = 0; v < 2; v++ ) faces[surface[first + j]][v] += e[v];
             }
             int n = 0;
             const auto now = Clock::now();
@@ -217,8 +225,8 @@ namespace
                 r.state = state[i];
                 r.min = d.mm[0];
                 r.max = d.mm[1];
-                r.quads = state[i] == FN2_CHUNK_SURFACE ? hCounts[2 * d.p.buffer] : 0;
-                r.solidVoxels = state[i] == FN2_CHUNK_SURFACE ? hCounts[2 * d.p.buffer + 1]
+                r.quads = faces[i][0];
+                r.solidVoxels = state[i] == FN2_CHUNK_SURFACE ? faces[i][1]
                               : state[i] == FN2_CHUNK_SOLID ? (uint32_t)size * size * size : 0;
                 r.latencyMs = std::chrono::duration<double, std::milli>( now - d.p.tRequest ).count();
                 r.version = d.p.version;
@@ -244,8 +252,10 @@ namespace
         std::vector<float*> buffers;
         std::vector<int> freeBuffers;
         std::set<std::array<int32_t, 3>> registered;
-        uint32_t* dCounts = nullptr;
-        uint32_t* hCounts = nullptr;
+        // pinned: the partial face counts of each consumer launch of a poll
+        uint32_t* hFaces = nullptr;
+        fn2::FastDiv divSize{};
+        uint32_t* FacesOf( size_t first ) { return hFaces + first / fn2::kFaceJobs * fn2::kFaceEntries * 2; }
         hipStream_t stream = nullptr;
         uint32_t version = 1;
     };
