@@ -121,8 +121,9 @@ namespace fn2
         return e;
     }
 
-    hipError_t LaunchProgram( const GenArgs& a, const DeviceProgram* dp, hipStream_t stream, bool* specialised )
+    hipError_t LaunchProgram( const GenArgs& a, const DeviceProgram* dp, hipStream_t stream, int32_t* direct, unsigned* blocks )
     {
+        if( blocks ) *blocks = 0;
         if( a.total <= 0 ) return hipSuccess;
         const int chosen = dp->variant.load( std::memory_order_relaxed );
         const JitKernel* k = GetJitKernel( dp );
@@ -134,13 +135,14 @@ namespace fn2
             if( const JitKernel* v = GetJitKernel( dp, chosen | kJitSharedWalk ) ) k = v;
         if( k )
         {
-            if( specialised ) *specialised = true;
             GenArgs copy = a;
             void* params[] = { &copy };
-            return hipModuleLaunchKernel( k->single, fn2_grid_for( a.total, k->blocksPerCU ), 1, 1, 256, 1, 1, 0, stream, params, nullptr );
+            const unsigned grid = fn2_grid_for( a.total, k->blocksPerCU );
+            if( blocks ) *blocks = grid;
+            if( direct && grid <= (unsigned)kRangeDirectBlocks ) copy.minmax = direct;
+            return hipModuleLaunchKernel( k->single, grid, 1, 1, 256, 1, 1, 0, stream, params, nullptr );
         }
-        if( specialised ) *specialised = false;
-        return (hipError_t)fn2_launch_generate( &a, dp->dimMask, dp->featMask, stream );
+        return (hipError_t)fn2_launch_generate( &a, dp->dimMask, dp->featMask, stream, direct, blocks );
     }
 
     FastDiv MakeFastDiv( uint32_t d )
@@ -323,8 +325,8 @@ namespace fn2
         }
         CallContext* c = new CallContext;
         if( !HipOk( hipStreamCreateWithFlags( &c->stream, hipStreamNonBlocking ), "hipStreamCreate" ) ||
-            !HipOk( hipMalloc( (void**)&c->dKeys, kCallRangeInts * sizeof( int32_t ) ), "hipMalloc(min/max)" ) ||
-            !HipOk( hipHostMalloc( (void**)&c->hKeys, kCallRangeInts * sizeof( int32_t ), hipHostMallocDefault ), "hipHostMalloc" ) ||
+            !HipOk( hipMalloc( (void**)&c->dKeys, kMaxCallBlocks * 2 * sizeof( int32_t ) ), "hipMalloc(min/max)" ) ||
+            !HipOk( hipHostMalloc( (void**)&c->hKeys, kRangeDirectBlocks * 2 * sizeof( int32_t ), hipHostMallocDefault ), "hipHostMalloc" ) ||
             !HipOk( hipEventCreate( &c->ev0 ), "hipEventCreate" ) || !HipOk( hipEventCreate( &c->ev1 ), "hipEventCreate" ) )
         {
             return nullptr;
@@ -337,6 +339,24 @@ namespace fn2
         if( !c ) return;
         std::lock_guard<std::mutex> lk( gMu );
         gContexts.push_back( c );
+    }
+
+    bool CallContext::LaunchRanged( GenArgs& a, const DeviceProgram* dp, hipStream_t st )
+    {
+        unsigned blocks = 0;
+        a.minmax = dKeys;
+        if( !HipOk( LaunchProgram( a, dp, st, hKeys, &blocks ), "launch generator" ) ) return false;
+        rangePairs = (int)blocks;
+        if( blocks <= (unsigned)kRangeDirectBlocks ) return true;
+        rangePairs = 1;
+        return HipOk( (hipError_t)fn2_launch_range_reduce( nullptr, { dKeys, (int32_t)blocks }, 1, hKeys, st ), "launch range reduction" );
+    }
+
+    void CallContext::Range( float& min, float& max ) const
+    {
+        if( DecodeRange( hKeys, rangePairs, 2, min, max ) ) return;
+        min = FastNoise::kInfinity;
+        max = -FastNoise::kInfinity;
     }
 
     bool CallContext::Reserve( float*& buf, size_t& cap, size_t floats )
@@ -537,8 +557,7 @@ namespace fn2
 
     bool FillSpecArgs( const fn2GenSpec& s, GenArgs& a, int64_t& total, std::string& err, const float* tileTable )
     {
-        a.rangeStride = kRangeStrideSpread;   // single calls; the serving engine packs its records
-        a.rangeSlots = kCallRangeSlots;
+        a.rangeSlots = kRangePerBlock;
         a.kind = s.kind;
         a.dims = s.dims;
         a.seed = s.seed;
@@ -641,7 +660,6 @@ namespace fn2
         a.regs = dp->regs;
         a.nIns = (int32_t)dp->ins.size();
         a.resultReg = dp->resultReg;
-        a.minmax = c->dKeys;
 
         const bool devOut = IsDevicePointer( out );
         if( devOut ) a.out = out;
@@ -678,9 +696,7 @@ namespace fn2
             }
         }
 
-        if( !HipOk( (hipError_t)fn2_launch_minmax_init( c->dKeys, 1, kCallRangeSlots, kRangeStrideSpread, c->stream ), "launch min/max init" ) ) return fail( tLastError );
-        if( !HipOk( LaunchProgram( a, dp, c->stream, nullptr ), "launch generator" ) ) return fail( tLastError );
-        if( !HipOk( hipMemcpyAsync( c->hKeys, c->dKeys, kCallRangeInts * sizeof( int32_t ), hipMemcpyDeviceToHost, c->stream ), "read min/max" ) ) return fail( tLastError );
+        if( !c->LaunchRanged( a, dp, c->stream ) ) return fail( tLastError );
         if( !devOut )
         {
             if( total >= kStagedMinFloats )
@@ -694,11 +710,7 @@ namespace fn2
         }
         if( !HipOk( hipStreamSynchronize( c->stream ), "generator kernel" ) ) return fail( tLastError );
 
-        if( !DecodeRange( c->hKeys, kCallRangeSlots, kRangeStrideSpread, r.min, r.max ) )
-        {
-            r.min = FastNoise::kInfinity;
-            r.max = -FastNoise::kInfinity;
-        }
+        c->Range( r.min, r.max );
         return r;
     }
 }
@@ -924,20 +936,15 @@ FASTNOISE_API int fn2GenerateDevice( const void* node, const fn2GenSpec* spec, f
     a.nIns = (int32_t)dp->ins.size();
     a.resultReg = dp->resultReg;
     a.out = dOut;
-    a.minmax = outputMinMax ? c->dKeys : nullptr;
-    if( outputMinMax && !HipOk( (hipError_t)fn2_launch_minmax_init( c->dKeys, 1, kCallRangeSlots, kRangeStrideSpread, st ), "launch min/max init" ) ) return 1;
-    if( !HipOk( LaunchProgram( a, dp, st, nullptr ), "launch generator" ) ) return 1;
     if( outputMinMax )
     {
-        if( !HipOk( hipMemcpyAsync( c->hKeys, c->dKeys, kCallRangeInts * sizeof( int32_t ), hipMemcpyDeviceToHost, st ), "read min/max" ) ) return 1;
+        if( !c->LaunchRanged( a, dp, st ) ) return 1;
         if( !HipOk( hipStreamSynchronize( st ), "generator kernel" ) ) return 1;
-        if( !DecodeRange( c->hKeys, kCallRangeSlots, kRangeStrideSpread, outputMinMax[0], outputMinMax[1] ) )
-        {
-            outputMinMax[0] = FastNoise::kInfinity;
-            outputMinMax[1] = -FastNoise::kInfinity;
-        }
+        c->Range( outputMinMax[0], outputMinMax[1] );
+        return 0;
     }
-    else if( !stream )
+    if( !HipOk( LaunchProgram( a, dp, st ), "launch generator" ) ) return 1;
+    if( !stream )
     {
         // the library stream belongs to the context that is released below:
         // finish the work before another call can pick it up
@@ -966,23 +973,18 @@ FASTNOISE_API int fn2BenchGenerate( const void* node, const fn2GenSpec* spec, fl
     a.nIns = (int32_t)dp->ins.size();
     a.resultReg = dp->resultReg;
     a.out = dOut;
+    // the range is part of the launch, its reduction is not
     a.minmax = c->dKeys;
     for( int i = 0; i < warmup; i++ )
     {
-        if( !HipOk( (hipError_t)fn2_launch_minmax_init( c->dKeys, 1, kCallRangeSlots, kRangeStrideSpread, c->stream ), "launch" ) ) return 1;
-        if( !HipOk( LaunchProgram( a, dp, c->stream, nullptr ), "launch" ) ) return 1;
+        if( !HipOk( LaunchProgram( a, dp, c->stream ), "launch" ) ) return 1;
     }
     if( !HipOk( hipStreamSynchronize( c->stream ), "warmup" ) ) return 1;
-    // The range keys are reset once: every timed launch writes the same
-    // output, so the keys accumulate the same min/max, and the timed region
-    // holds generator launches only.
-    if( !HipOk( (hipError_t)fn2_launch_minmax_init( c->dKeys, 1, kCallRangeSlots, kRangeStrideSpread, c->stream ), "launch" ) ) return 1;
-    if( !HipOk( hipStreamSynchronize( c->stream ), "range reset" ) ) return 1;
     auto t0 = std::chrono::steady_clock::now();
     if( !HipOk( hipEventRecord( c->ev0, c->stream ), "event" ) ) return 1;
     for( int i = 0; i < iters; i++ )
     {
-        if( !HipOk( LaunchProgram( a, dp, c->stream, nullptr ), "launch" ) ) return 1;
+        if( !HipOk( LaunchProgram( a, dp, c->stream ), "launch" ) ) return 1;
     }
     if( !HipOk( hipEventRecord( c->ev1, c->stream ), "event" ) ) return 1;
     if( !HipOk( hipStreamSynchronize( c->stream ), "timed launches" ) ) return 1;

@@ -46,11 +46,18 @@ namespace fn2
         size_t outCap = 0;
         float* dPos = nullptr;
         size_t posCap = 0;
-        int32_t* dKeys = nullptr;   // one range record, slots kRangeStrideSpread ints apart
-        int32_t* hKeys = nullptr;   // pinned, the same size
+        int32_t* dKeys = nullptr;   // a call's range record: kMaxCallBlocks pairs
+        int32_t* hKeys = nullptr;   // pinned: kRangeDirectBlocks pairs, written by the kernels
         hipEvent_t ev0 = nullptr, ev1 = nullptr;
         float* hStage = nullptr;    // pinned ring: kStageSlots chunks of kStageChunkFloats
         hipEvent_t evStage[kStageSlots] = {};
+
+        // A ranged launch on `st`: the generator with its range record, and
+        // the record's reduction where it takes one; after the stream has
+        // been waited for, Range gives the result of the last one
+        bool LaunchRanged( GenArgs& a, const DeviceProgram* dp, hipStream_t st );
+        void Range( float& min, float& max ) const;
+        int rangePairs = 0;
 
         bool Reserve( float*& buf, size_t& cap, size_t floats );
         bool ReserveStage();
@@ -80,7 +87,7 @@ namespace fn2
     // The range a record holds: false when no number was published to it
     // (every output NaN, or none), else its min and max
     bool DecodeRange( const int32_t* record, int slots, int stride, float& min, float& max );
-    // ints of a single call's range record
+    // ints of the record of slots of the entry point that allocates nothing
     constexpr int kCallRangeInts = kCallRangeSlots * kRangeStrideSpread;
     // Launch arguments of a spec (everything but the program and the output).
     // A tileable spec uses `tileTable` (device floats laid out as FillTileTable
@@ -101,8 +108,11 @@ namespace fn2
     bool CompileForDevice( const FastNoise::Generator* root, int dims, const DeviceProgram*& dp, Program* hostCopy );
 
     // One generator launch: the tree's specialised kernel when it is loaded,
-    // the interpreter otherwise (`specialised` reports which).
-    hipError_t LaunchProgram( const GenArgs& a, const DeviceProgram* dp, hipStream_t stream, bool* specialised );
+    // the interpreter otherwise. A range record is made the caller's: of a
+    // pair per block in `direct` (pinned) when the launch has at most
+    // kRangeDirectBlocks blocks, else in a.minmax. `blocks` receives the
+    // launch's blocks.
+    hipError_t LaunchProgram( const GenArgs& a, const DeviceProgram* dp, hipStream_t stream, int32_t* direct = nullptr, unsigned* blocks = nullptr );
 
     CallContext* AcquireContext();
     void ReleaseContext( CallContext* c );

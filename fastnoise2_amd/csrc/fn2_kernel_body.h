@@ -4,11 +4,9 @@
 // returns its value: either the interpreter loop or a fixed, inlined program.
 //
 // Output range: every lane keeps a running min/max in registers; a block
-// reduces them through wave shuffles and LDS and publishes one atomic pair.
-// Same-address atomics serialise in L2, so the number of blocks, not of
-// waves, bounds their cost: the single-call kernel runs a grid-stride loop
-// over a grid sized to fill the GPU, and the batched kernel gives each block
-// a tile of several points per lane.
+// reduces them through wave shuffles and LDS and stores its pair (or, into a
+// record of slots, publishes one atomic pair; same-address atomics serialise
+// in L2, so the number of blocks, not of waves, bounds their cost).
 #pragma once
 #include "fn2_interp.h"
 
@@ -25,9 +23,8 @@ namespace fn2k
     // BLOCK: the most threads a block of the kernel has (its launch bound);
     // the block may have fewer, any multiple of 64.
     template<int BLOCK>
-    __device__ __forceinline__ void blockMinMax( float mn, float mx, int32_t* record, int stride, int slots )
+    __device__ __forceinline__ void blockMinMax( float mn, float mx, int32_t* record, int stride, int slots, uint32_t block )
     {
-        int32_t* keys = record + ( blockIdx.x & (uint32_t)( slots - 1 ) ) * stride;
         __shared__ float sMin[BLOCK / 64], sMax[BLOCK / 64];
 #pragma unroll
         for( int off = 32; off > 0; off >>= 1 )
@@ -52,8 +49,17 @@ namespace fn2k
                 mn = fminf( mn, sMin[w] );
                 mx = fmaxf( mx, sMax[w] );
             }
-            if( mn <= mx )
+            if( slots == fn2::kRangePerBlock )
             {
+                // the block's own pair; a block without a number stores the empty one
+                int2 pair;
+                pair.x = mn <= mx ? orderedKey( mn ) : 0x7fffffff;
+                pair.y = mn <= mx ? orderedKey( mx ) : (int32_t)0x80000000u;
+                reinterpret_cast<int2*>( record )[block] = pair;
+            }
+            else if( mn <= mx )
+            {
+                int32_t* keys = record + ( block & (uint32_t)( slots - 1 ) ) * stride;
                 atomicMin( &keys[0], orderedKey( mn ) );
                 atomicMax( &keys[1], orderedKey( mx ) );
             }
@@ -187,7 +193,7 @@ namespace fn2k
                 emit( i, prog( a, R ) );
             }
         }
-        if( a.minmax ) blockMinMax<BLOCK>( mn, mx, a.minmax, a.rangeStride, a.rangeSlots );
+        if( a.minmax ) blockMinMax<BLOCK>( mn, mx, a.minmax, a.rangeStride, a.rangeSlots, blockIdx.x );
     }
 
     // One tile of a batched request: points [first, first + threads * ppt)
@@ -239,7 +245,8 @@ namespace fn2k
                 }
             }
         }
-        if( a.minmax ) blockMinMax<BLOCK>( mn, mx, a.minmax, a.rangeStride, a.rangeSlots );
+        // the job's block: its tiles start at multiples of their size
+        if( a.minmax ) blockMinMax<BLOCK>( mn, mx, a.minmax, a.rangeStride, a.rangeSlots, first / ( threads * (uint32_t)ppt ) );
     }
 
     // Batched requests: block b runs tile (blockJob[b], blockBase[b]).

@@ -8,13 +8,8 @@
 // GPR indexing, no scratch) and writes one float with a coalesced store.
 //
 // Output range: every lane keeps a running min/max in registers; a block
-// reduces them through wave shuffles and LDS and publishes one atomic pair
-// to the slot of its index in the call's range record (fn2_kernel_args.h).
-// Same-address atomics queue one behind the other, so the slots spread them;
-// the number of blocks still bounds their cost: the single-call kernel runs a
-// grid-stride loop over a grid sized to fill the GPU (a few thousand
-// blocks), and the batched kernel gives each block a tile of several points
-// per lane.
+// reduces them through wave shuffles and LDS and stores its pair to the
+// call's range record (fn2_kernel_args.h).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <algorithm>
@@ -123,6 +118,41 @@ __global__ void __launch_bounds__( 256 ) fn2_bloxel_faces( fn2::FaceJobs jobs, i
         partials[blockIdx.y * gridDim.x + blockIdx.x] = make_uint2( sq[0] + sq[1] + sq[2] + sq[3], ss[0] + ss[1] + ss[2] + ss[3] );
 }
 
+// Reduces range records of a pair per block: block j takes record j (of
+// `one` when jobs is null) and writes its pair to out + 2 j, in pinned host
+// memory. A launch-sized kernel: 8192 pairs are 8 loads per thread.
+__global__ void __launch_bounds__( 1024 ) fn2_range_reduce( const fn2::GenArgs* __restrict__ jobs, fn2::RangeRecord one, int32_t* __restrict__ out )
+{
+    if( jobs ) one = { jobs[blockIdx.x].minmax, jobs[blockIdx.x].rangeStride };
+    int32_t mn = 0x7fffffff, mx = (int32_t)0x80000000u;
+    const int2* pairs = reinterpret_cast<const int2*>( one.pairs );
+    for( int i = threadIdx.x; i < one.count; i += 1024 )
+    {
+        const int2 p = pairs[i];
+        mn = min( mn, p.x );
+        mx = max( mx, p.y );
+    }
+    __shared__ int2 part[16];
+#pragma unroll
+    for( int off = 32; off > 0; off >>= 1 )
+    {
+        mn = min( mn, __shfl_xor( mn, off ) );
+        mx = max( mx, __shfl_xor( mx, off ) );
+    }
+    if( ( threadIdx.x & 63 ) == 0 ) part[threadIdx.x >> 6] = make_int2( mn, mx );
+    __syncthreads();
+    if( threadIdx.x == 0 )
+    {
+#pragma unroll
+        for( int w = 1; w < 16; w++ )
+        {
+            mn = min( mn, part[w].x );
+            mx = max( mx, part[w].y );
+        }
+        reinterpret_cast<int2*>( out )[blockIdx.x] = make_int2( mn, mx );
+    }
+}
+
 // Resets n consecutive range records (`slots` slots each, `stride` ints
 // apart) and zeroes nc work-queue counters
 __global__ void fn2_minmax_init( int32_t* keys, int n, int slots, int stride, uint32_t* counters, int nc )
@@ -173,11 +203,11 @@ namespace
         if( blocksPerCU <= 0 )
         {
             const int64_t need = ( total + kBlock - 1 ) / kBlock;
-            const int64_t cap = (int64_t)CUs() * 16;
+            const int64_t cap = std::min<int64_t>( (int64_t)CUs() * 16, fn2::kMaxCallBlocks );
             return (unsigned)( need < cap ? need : cap );
         }
         const int64_t need = std::max<int64_t>( 1, ( total + kBlock - 1 ) / kBlock );
-        const int64_t cap = (int64_t)CUs() * blocksPerCU * rounds;
+        const int64_t cap = std::min<int64_t>( (int64_t)CUs() * blocksPerCU * rounds, fn2::kMaxCallBlocks );
         return (unsigned)( need < cap ? need : cap );
     }
 
@@ -233,8 +263,9 @@ int fn2_batch_block_threads( void )
     return kBlock;
 }
 
-int fn2_launch_generate( const fn2::GenArgs* args, int dimMask, int featMask, hipStream_t stream )
+int fn2_launch_generate( const fn2::GenArgs* args, int dimMask, int featMask, hipStream_t stream, int32_t* direct, unsigned* blocks )
 {
+    if( blocks ) *blocks = 0;
     if( args->total <= 0 ) return 0;
     // the register file in LDS: one column of args->regs floats per thread
     if( args->regs < 1 || args->regs > fn2::kMaxRegs ) return (int)hipErrorInvalidValue;
@@ -245,7 +276,10 @@ int fn2_launch_generate( const fn2::GenArgs* args, int dimMask, int featMask, hi
         static std::atomic<int> resident[fn2::kMaxRegs + 1];   /* per register count, zero at start */ \
         const int bpc = CachedResident( resident, args->regs, fn2_generate<kBlock, DMV, FTV>, lds ); \
         const unsigned grid = GridFor( args->total, bpc, 4 ); \
-        hipLaunchKernelGGL( ( fn2_generate<kBlock, DMV, FTV> ), dim3( grid ), dim3( kBlock ), lds, stream, *args ); \
+        if( blocks ) *blocks = grid; \
+        fn2::GenArgs copy = *args; \
+        if( direct && grid <= (unsigned)fn2::kRangeDirectBlocks ) copy.minmax = direct; \
+        hipLaunchKernelGGL( ( fn2_generate<kBlock, DMV, FTV> ), dim3( grid ), dim3( kBlock ), lds, stream, copy ); \
         return (int)hipGetLastError(); \
     }
     FN2_VARIANTS( FN2_TRY )
@@ -323,6 +357,14 @@ int fn2_launch_bloxel_faces( const fn2::FaceJobs* jobs, int n, int gen, fn2::Fas
     for( int i = 0; i < n; i++ )
         if( !jobs->density[i] ) return (int)hipErrorInvalidValue;
     hipLaunchKernelGGL( fn2_bloxel_faces, dim3( fn2_face_blocks( n, gen ), n ), dim3( 256 ), 0, stream, *jobs, gen, divS, iso, (uint2*)partials );
+    return (int)hipGetLastError();
+}
+
+int fn2_launch_range_reduce( const fn2::GenArgs* dJobs, fn2::RangeRecord one, int n, int32_t* out, hipStream_t stream )
+{
+    if( n <= 0 ) return 0;
+    if( !out || ( !dJobs && ( n != 1 || !one.pairs ) ) ) return (int)hipErrorInvalidValue;
+    hipLaunchKernelGGL( fn2_range_reduce, dim3( n ), dim3( 1024 ), 0, stream, dJobs, one, out );
     return (int)hipGetLastError();
 }
 

@@ -8,6 +8,13 @@
 
 namespace fn2
 {
+    // A range record of a pair per block
+    struct RangeRecord
+    {
+        const int32_t* pairs;
+        int32_t count;
+    };
+
     // Density blocks of one face-count launch, passed by value, and the
     // { quads, solid } entries its blocks write at most
     // (fn2_face_blocks( n, gen ) per chunk, n <= kFaceJobs)
@@ -20,10 +27,12 @@ namespace fn2
 }
 
 extern "C" {
-// one interpreter launch over args->total points
-int fn2_launch_generate( const fn2::GenArgs* args, int dimMask, int featMask, hipStream_t stream );
+// one interpreter launch over args->total points. `blocks` (may be null)
+// receives the launch's blocks; with at most kRangeDirectBlocks of them their
+// range pairs go to `direct` (unless null) instead of args->minmax
+int fn2_launch_generate( const fn2::GenArgs* args, int dimMask, int featMask, hipStream_t stream, int32_t* direct, unsigned* blocks );
 // blocks of a single-call launch over `total` points (also used for the
-// run-time specialised kernels)
+// run-time specialised kernels), at most kMaxCallBlocks
 unsigned fn2_grid_for( int64_t total, int blocksPerCU );
 // interpreter launch over a batch of jobs (block b runs job dBlockJob[b])
 int fn2_launch_generate_batch( const fn2::GenArgs* dJobs, const int32_t* dBlockJob, const uint32_t* dBlockBase, int nBlocks, int dimMask, int featMask,
@@ -31,6 +40,9 @@ int fn2_launch_generate_batch( const fn2::GenArgs* dJobs, const int32_t* dBlockJ
 // interpreter work-queue launch over nTiles tiles of a batch
 int fn2_launch_generate_queue( const fn2::GenArgs* dJobs, const int32_t* dTileJob, const uint32_t* dTileBase, int nTiles, int dimMask, int featMask,
                                int regs, uint32_t* dCounter, hipStream_t stream );
+// reduces n per-block range records (those of dJobs, or `one` when dJobs is
+// null) to a pair each at out + 2 j
+int fn2_launch_range_reduce( const fn2::GenArgs* dJobs, fn2::RangeRecord one, int n, int32_t* out, hipStream_t stream );
 // resets n consecutive range records of `slots` slots, `stride` ints apart
 int fn2_launch_minmax_init( int32_t* keys, int n, int slots, int stride, hipStream_t stream );
 // the same, also zeroing nc work-queue counters

@@ -182,6 +182,8 @@ FASTNOISE_API int fn2GenerateDeviceNoAlloc( const void* node, const fn2GenSpec* 
     a.resultReg = p.resultReg;
     a.out = dOut;
     a.minmax = outputMinMax ? dKeys : nullptr;
+    a.rangeStride = kRangeStrideSpread;
+    a.rangeSlots = kCallRangeSlots;
     // the range record starts empty: a fill kernel, not a memset, so that the
     // call can be recorded into a graph
     if( outputMinMax && !HipOk( (hipError_t)fn2_launch_minmax_init( dKeys, 1, kCallRangeSlots, kRangeStrideSpread, st ), "launch min/max init" ) ) return 1;
@@ -193,7 +195,7 @@ FASTNOISE_API int fn2GenerateDeviceNoAlloc( const void* node, const fn2GenSpec* 
                     "launch specialised generator" ) )
             return 1;
     }
-    else if( !HipOk( (hipError_t)fn2_launch_generate( &a, p.dimMask, p.featMask, st ), "launch generator" ) ) return 1;
+    else if( !HipOk( (hipError_t)fn2_launch_generate( &a, p.dimMask, p.featMask, st, nullptr, nullptr ), "launch generator" ) ) return 1;
     if( outputMinMax )
     {
         int32_t keys[kCallRangeInts];

@@ -4,11 +4,12 @@
 // fn2ServeSubmit from any thread. A dispatcher thread admits queued requests
 // FIFO into the next free batch slot as long as the slot's point capacity
 // allows, writes one job record per request (GenArgs pointing at the
-// request's output range in the slot's device arena and at its own min/max
-// key pair) plus a block -> (job, first point) table, and launches the batch
+// request's output range in the slot's device arena and at its own range
+// record) plus a block -> (job, first point) table, and launches the batch
 // kernel once per kernel variant present in the batch, followed by the copy
-// of the slot's outputs and keys into pinned host memory (requests into
-// device memory have theirs as the output range). Slots run on their
+// of the slot's outputs into pinned host memory (requests into device memory
+// have theirs as the output range; the blocks' ranges go straight to pinned
+// memory). Slots run on their
 // own streams, so a batch formed from requests that arrived while the
 // previous one was on the GPU overlaps with it. A completion thread retires
 // slots in launch order: it copies each request's values into the caller's
@@ -58,8 +59,6 @@ namespace
 
     // threads per block of the batched kernel; requests start on multiples of it
     const int kThreads = fn2_batch_block_threads();
-    // the tuner's range record: compact
-    constexpr int kTuneRangeInts = fn2::kRangeSlots * fn2::kRangeStrideCompact;
     // the tuner's candidates: points per lane, threads per block (the
     // specialised batch kernel; the interpreter's register file in LDS is laid
     // out for kThreads), and its calibration size
@@ -111,6 +110,7 @@ namespace
         // placement in its batch slot
         size_t outOffset = 0;
         int job = 0;
+        int firstBlock = 0, blocks = 0;   // its pairs in the slot's range record
         int ppt = 1;
         int threads = 256;   // threads per block when a specialised kernel runs it
         int variant = 0;     // variant of the specialised kernel
@@ -137,14 +137,20 @@ namespace
         hipEvent_t done = nullptr;
         float* dOut = nullptr;          // capacity floats
         float* hOut = nullptr;          // pinned
-        int32_t* dKeys = nullptr;       // a range record per job, then the persistent mode's work counters (kQueueCounterInts per launch)
+        // range records: a pair per block of the batch in device memory, and
+        // in pinned memory the blocks' pairs of a small batch or the jobs'
+        // pairs of a larger one
+        int32_t* dRange = nullptr;
+        int32_t* hRange = nullptr;
+        bool rangeDirect = false;
+        // persistent mode instead: a range record of slots per job, then the
+        // work counters (kQueueCounterInts per launch)
+        int32_t* dKeys = nullptr;
         uint32_t* dCounter = nullptr;
         int32_t* hKeys = nullptr;       // pinned
-        GenArgs* dJobs = nullptr;
-        int32_t* dBlockJob = nullptr;
-        uint32_t* dBlockBase = nullptr;
-        uint8_t* hTables = nullptr;     // pinned: jobs | blockJob | blockBase
-        size_t tableBytes = 0;
+        // jobs | blockJob | blockBase, packed for the batch at hand
+        uint8_t* dTables = nullptr;
+        uint8_t* hTables = nullptr;     // pinned
         std::vector<Request*> reqs;
         int64_t points = 0;
         bool busy = false;
@@ -164,33 +170,26 @@ namespace
     {
     public:
         int mode;
-        int jobStride = fn2::kRangeStrideCompact;   // ints between a request's range slots
-        int jobRangeInts = fn2::kRangeSlots * fn2::kRangeStrideCompact;
+        // persistent mode: ints of a request's range record. Its kernels
+        // publish a range per wave (four times as many atomics as blocks),
+        // which queue up within one line, so a slot has a line
+        const int jobRangeInts = fn2::kRangeSlots * fn2::kRangeStrideSpread;
         int64_t capacity;       // points per batch
         size_t budget;
         std::string initError;
 
-        Engine( size_t hbmBudget, int maxBatchPoints, int m ) : mode( m ), capacity( maxBatchPoints ), budget( hbmBudget )
-        {
-            // A request's range record: the engine reads one back per
-            // request, so compact; the work-queue kernels publish a range per
-            // wave (four times as many atomics as a block-per-tile launch),
-            // which queue up within one line, so they get a line per slot
-            jobStride = mode == FN2_SERVE_PERSISTENT ? fn2::kRangeStrideSpread : fn2::kRangeStrideCompact;
-            jobRangeInts = fn2::kRangeSlots * jobStride;
-        }
+        Engine( size_t hbmBudget, int maxBatchPoints, int m ) : mode( m ), capacity( maxBatchPoints ), budget( hbmBudget ) {}
 
         bool Init()
         {
             if( capacity < kThreads ) capacity = kThreads;
             capacity = (int64_t)AlignUp( (size_t)capacity, kThreads );
             maxBlocks = (int)( capacity / kThreadCandidates[0] ) + kMaxJobs;   // the smallest tiles
-            size_t jobsBytes = AlignUp( sizeof( GenArgs ) * kMaxJobs, 256 );
-            size_t bjBytes = AlignUp( sizeof( int32_t ) * maxBlocks, 256 );
-            size_t bbBytes = AlignUp( sizeof( uint32_t ) * maxBlocks, 256 );
-            // range records, then (persistent mode) the counters of up to a launch per job
-            const size_t keyBytes = ( jobRangeInts + ( mode == FN2_SERVE_PERSISTENT ? fn2::kQueueCounterInts : 0 ) ) * sizeof( int32_t ) * kMaxJobs;
-            size_t perSlot = (size_t)capacity * 4 + jobsBytes + bjBytes + bbBytes + keyBytes;
+            const size_t tableBytes = Tables( kMaxJobs, maxBlocks ).bytes;
+            // persistent mode: range records, then the counters of up to a launch per job
+            const size_t keyBytes = mode == FN2_SERVE_PERSISTENT ? (size_t)( jobRangeInts + fn2::kQueueCounterInts ) * sizeof( int32_t ) * kMaxJobs : 0;
+            const size_t rangeBytes = mode == FN2_SERVE_PERSISTENT ? 0 : (size_t)maxBlocks * 2 * sizeof( int32_t );
+            size_t perSlot = (size_t)capacity * 4 + tableBytes + keyBytes + rangeBytes;
             int nSlots = mode == FN2_SERVE_PLAIN ? 1 : kSlots;
             if( perSlot * nSlots > budget )
             {
@@ -200,22 +199,21 @@ namespace
             slots.resize( nSlots );
             for( Slot& s : slots )
             {
-                s.tableBytes = jobsBytes + bjBytes + bbBytes;
                 if( !fn2::HipOk( hipStreamCreateWithFlags( &s.stream, hipStreamNonBlocking ), "serve stream" ) ||
                     !fn2::HipOk( hipEventCreateWithFlags( &s.done, hipEventDisableTiming ), "serve event" ) ||
                     !fn2::HipOk( hipMalloc( (void**)&s.dOut, (size_t)capacity * 4 ), "serve arena" ) ||
                     !fn2::HipOk( hipHostMalloc( (void**)&s.hOut, (size_t)capacity * 4, hipHostMallocDefault ), "serve staging" ) ||
-                    !fn2::HipOk( hipMalloc( (void**)&s.dKeys, keyBytes ), "serve keys" ) ||
-                    !fn2::HipOk( hipHostMalloc( (void**)&s.hKeys, keyBytes, hipHostMallocDefault ), "serve keys" ) ||
-                    !fn2::HipOk( hipMalloc( (void**)&s.dJobs, s.tableBytes ), "serve tables" ) ||
-                    !fn2::HipOk( hipHostMalloc( (void**)&s.hTables, s.tableBytes, hipHostMallocDefault ), "serve tables" ) )
+                    ( rangeBytes && !fn2::HipOk( hipMalloc( (void**)&s.dRange, rangeBytes ), "serve ranges" ) ) ||
+                    !fn2::HipOk( hipHostMalloc( (void**)&s.hRange, (size_t)std::max( kMaxJobs, fn2::kRangeDirectBlocks ) * 2 * sizeof( int32_t ), hipHostMallocDefault ), "serve ranges" ) ||
+                    ( keyBytes && !fn2::HipOk( hipMalloc( (void**)&s.dKeys, keyBytes ), "serve keys" ) ) ||
+                    ( keyBytes && !fn2::HipOk( hipHostMalloc( (void**)&s.hKeys, keyBytes, hipHostMallocDefault ), "serve keys" ) ) ||
+                    !fn2::HipOk( hipMalloc( (void**)&s.dTables, tableBytes ), "serve tables" ) ||
+                    !fn2::HipOk( hipHostMalloc( (void**)&s.hTables, tableBytes, hipHostMallocDefault ), "serve tables" ) )
                 {
                     initError = fn2::LastError();
                     return false;
                 }
-                s.dCounter = (uint32_t*)( s.dKeys + (size_t)jobRangeInts * kMaxJobs );
-                s.dBlockJob = (int32_t*)( (uint8_t*)s.dJobs + jobsBytes );
-                s.dBlockBase = (uint32_t*)( (uint8_t*)s.dJobs + jobsBytes + bjBytes );
+                if( keyBytes ) s.dCounter = (uint32_t*)( s.dKeys + (size_t)jobRangeInts * kMaxJobs );
             }
             deviceBytes = (int64_t)( perSlot * nSlots );
             {
@@ -235,13 +233,13 @@ namespace
                     !fn2::HipOk( hipEventCreate( &tuneEv0 ), "tune event" ) || !fn2::HipOk( hipEventCreate( &tuneEv1 ), "tune event" ) ||
                     !fn2::HipOk( hipMalloc( (void**)&tuneOut, (size_t)kTunePoints * 4 ), "tune arena" ) ||
                     !fn2::HipOk( hipMalloc( (void**)&tuneJob, sizeof( GenArgs ) ), "tune job" ) ||
-                    !fn2::HipOk( hipMalloc( (void**)&tuneKeys, kTuneRangeInts * sizeof( int32_t ) ), "tune keys" ) ||
+                    !fn2::HipOk( hipMalloc( (void**)&tuneKeys, tb * 2 * sizeof( int32_t ) ), "tune keys" ) ||
                     !fn2::HipOk( hipMalloc( (void**)&tuneBJ, tb * sizeof( int32_t ) * 2 ), "tune tables" ) )
                 {
                     initError = fn2::LastError();
                     return false;
                 }
-                deviceBytes += (int64_t)( (size_t)kTunePoints * 4 + sizeof( GenArgs ) + kTuneRangeInts * 4 + tb * 8 );
+                deviceBytes += (int64_t)( (size_t)kTunePoints * 4 + sizeof( GenArgs ) + tb * 16 );
             }
             copies.reset( new fn2::CopyPool( 3 ) );
             dispatcher = std::thread( [this] { DispatchLoop(); } );
@@ -267,9 +265,11 @@ namespace
                 if( s.graph ) (void)hipGraphDestroy( s.graph );
                 if( s.dOut ) (void)hipFree( s.dOut );
                 if( s.hOut ) (void)hipHostFree( s.hOut );
+                if( s.dRange ) (void)hipFree( s.dRange );
+                if( s.hRange ) (void)hipHostFree( s.hRange );
                 if( s.dKeys ) (void)hipFree( s.dKeys );
                 if( s.hKeys ) (void)hipHostFree( s.hKeys );
-                if( s.dJobs ) (void)hipFree( s.dJobs );
+                if( s.dTables ) (void)hipFree( s.dTables );
                 if( s.hTables ) (void)hipHostFree( s.hTables );
                 if( s.done ) (void)hipEventDestroy( s.done );
                 if( s.stream ) (void)hipStreamDestroy( s.stream );
@@ -677,9 +677,7 @@ namespace
             a.nIns = (int32_t)prog->ins.size();
             a.resultReg = prog->resultReg;
             a.out = tuneOut;
-            a.minmax = tuneKeys;
-            a.rangeStride = fn2::kRangeStrideCompact;
-            a.rangeSlots = fn2::kRangeSlots;
+            a.minmax = tuneKeys;   // a pair per block, as batches have (FillSpecArgs)
             return true;
         }
 
@@ -709,8 +707,7 @@ namespace
                 const int32_t* bjp = dBJ;
                 const uint32_t* bbp = dBB;
                 void* params[] = { (void*)&jobs, (void*)&bjp, (void*)&bbp };
-                if( !fn2::HipOk( (hipError_t)fn2_launch_minmax_init( tuneKeys, 1, fn2::kRangeSlots, fn2::kRangeStrideCompact, tuneStream ), "tune launch" ) ||
-                    !fn2::HipOk( hipEventRecord( tuneEv0, tuneStream ), "tune event" ) ||
+                if( !fn2::HipOk( hipEventRecord( tuneEv0, tuneStream ), "tune event" ) ||
                     !fn2::HipOk( jit ? hipModuleLaunchKernel( jit->batch, (unsigned)nb, 1, 1, (unsigned)threads, 1, 1, 0, tuneStream, params, nullptr )
                                      : (hipError_t)fn2_launch_generate_batch( tuneJob, dBJ, dBB, nb, prog->dimMask, prog->featMask, prog->regs, tuneStream ),
                                  "tune launch" ) ||
@@ -800,11 +797,6 @@ namespace
                 const int64_t ka = KernelKey( a->prog, a->jit ), kb = KernelKey( b->prog, b->jit );
                 return ka != kb ? ka < kb : a->threads < b->threads;
             } );
-            GenArgs* hJobs = (GenArgs*)s.hTables;
-            size_t jobsBytes = AlignUp( sizeof( GenArgs ) * kMaxJobs, 256 );
-            size_t bjBytes = AlignUp( sizeof( int32_t ) * maxBlocks, 256 );
-            int32_t* hBJ = (int32_t*)( s.hTables + jobsBytes );
-            uint32_t* hBB = (uint32_t*)( s.hTables + jobsBytes + bjBytes );
             // (kernel key, blocks, register-file size, threads per block) per
             // launch; the register file (interpreter launches only) sizes the
             // launch's LDS
@@ -819,7 +811,20 @@ namespace
             for( size_t j = 0; j < order.size(); j++ )
             {
                 Request* r = order[j];
+                const int64_t tile = (int64_t)r->threads * std::min( r->ppt, pptCap );
                 r->job = (int)j;
+                r->firstBlock = nb;
+                r->blocks = (int)( ( r->points + tile - 1 ) / tile );
+                nb += r->blocks;
+            }
+            s.rangeDirect = nb <= fn2::kRangeDirectBlocks;
+            const Tables tables( (int)order.size(), nb );
+            GenArgs* hJobs = (GenArgs*)s.hTables;
+            int32_t* hBJ = (int32_t*)( s.hTables + tables.blockJob );
+            uint32_t* hBB = (uint32_t*)( s.hTables + tables.blockBase );
+            for( size_t j = 0; j < order.size(); j++ )
+            {
+                Request* r = order[j];
                 GenArgs a = r->args;
                 // Device destinations are the kernels' own output: a copy per
                 // request from the arena took about 3 us each in stream order.
@@ -829,16 +834,25 @@ namespace
                 a.out = r->dest == Request::kDirect ? r->hostOut : s.dOut + r->outOffset;
                 const int ppt = std::min( r->ppt, pptCap );
                 a.ppt = ppt;
-                a.minmax = s.dKeys + (size_t)jobRangeInts * j;
-                a.rangeStride = jobStride;
-                a.rangeSlots = fn2::kRangeSlots;
+                if( mode == FN2_SERVE_PERSISTENT )
+                {
+                    a.minmax = s.dKeys + (size_t)jobRangeInts * j;
+                    a.rangeStride = fn2::kRangeStrideSpread;
+                    a.rangeSlots = fn2::kRangeSlots;
+                }
+                else
+                {
+                    // a pair per block (FillSpecArgs)
+                    a.minmax = ( s.rangeDirect ? s.hRange : s.dRange ) + (size_t)2 * r->firstBlock;
+                    a.rangeStride = r->blocks;
+                }
                 hJobs[j] = a;
                 const int64_t tile = (int64_t)r->threads * ppt;
-                int rb = (int)( ( r->points + tile - 1 ) / tile );
+                const int rb = r->blocks;
                 for( int b = 0; b < rb; b++ )
                 {
-                    hBJ[nb + b] = (int32_t)j;
-                    hBB[nb + b] = (uint32_t)( b * tile );
+                    hBJ[r->firstBlock + b] = (int32_t)j;
+                    hBB[r->firstBlock + b] = (uint32_t)( b * tile );
                 }
                 int64_t key = KernelKey( r->prog, r->jit );
                 const int64_t regs = r->jit ? 0 : r->prog->regs;
@@ -852,7 +866,6 @@ namespace
                     shape.back()[1] += rb;
                     shape.back()[2] = std::max( shape.back()[2], regs );
                 }
-                nb += rb;
             }
             if( mode == FN2_SERVE_PERSISTENT )
             {
@@ -875,7 +888,6 @@ namespace
                 }
             }
             const int nJobs = (int)order.size();
-            // the blocks of the tables that are used: copy jobs, then block tables
             if( mode == FN2_SERVE_GRAPH )
             {
                 if( s.exec && ( s.graphJobs != nJobs || s.graphShape != shape ) )
@@ -907,34 +919,51 @@ namespace
             return true;
         }
 
+        // Where a batch's tables lie in the slot's table buffers, packed so
+        // that one copy uploads them: the job records at 0, then a job index
+        // and a first point per block
+        struct Tables
+        {
+            size_t blockJob, blockBase, bytes;
+            Tables( int jobs, int blocks )
+            {
+                blockJob = AlignUp( sizeof( GenArgs ) * jobs, 256 );
+                blockBase = blockJob + AlignUp( sizeof( int32_t ) * blocks, 256 );
+                bytes = blockBase + AlignUp( sizeof( uint32_t ) * blocks, 256 );
+            }
+        };
+
         // Stream work of one batch that depends only on its shape (recorded
-        // once per shape in graph mode): table upload, range-key reset, one
-        // batch launch per kernel.
+        // once per shape in graph mode): table upload, the persistent mode's
+        // range and counter reset, one batch launch per kernel. In the other
+        // modes the blocks' range pairs are reduced by a launch after them
+        // (small batches: read by the host). With one upload and no reset,
+        // a burst of 64 requests of the serving tree took 0.496 ms on MI355X,
+        // with three uploads, the reset and the copy of a record of slots
+        // per request 0.536.
         bool Enqueue( Slot& s, const std::vector<std::array<int64_t, 4>>& shape, const std::vector<const fn2::JitKernel*>& kernels,
                       int nJobs, int nb )
         {
-            size_t jobsBytes = AlignUp( sizeof( GenArgs ) * kMaxJobs, 256 );
-            size_t bjBytes = AlignUp( sizeof( int32_t ) * maxBlocks, 256 );
-            size_t usedJob = sizeof( GenArgs ) * nJobs;
-            if( !fn2::HipOk( hipMemcpyAsync( s.dJobs, s.hTables, usedJob, hipMemcpyHostToDevice, s.stream ), "upload jobs" ) ) return false;
-            if( !fn2::HipOk( hipMemcpyAsync( s.dBlockJob, s.hTables + jobsBytes, sizeof( int32_t ) * nb, hipMemcpyHostToDevice, s.stream ), "upload blocks" ) ) return false;
-            if( !fn2::HipOk( hipMemcpyAsync( s.dBlockBase, s.hTables + jobsBytes + bjBytes, sizeof( uint32_t ) * nb, hipMemcpyHostToDevice, s.stream ), "upload blocks" ) ) return false;
+            const Tables tables( nJobs, nb );
+            const fn2::GenArgs* jobs = (const fn2::GenArgs*)s.dTables;
+            const int32_t* blockJob = (const int32_t*)( s.dTables + tables.blockJob );
+            const uint32_t* blockBase = (const uint32_t*)( s.dTables + tables.blockBase );
+            if( !fn2::HipOk( hipMemcpyAsync( s.dTables, s.hTables, tables.bytes, hipMemcpyHostToDevice, s.stream ), "upload tables" ) ) return false;
             if( mode == FN2_SERVE_PERSISTENT )
             {
                 // range keys and one zero counter per work-queue launch, in one kernel
-                if( !fn2::HipOk( (hipError_t)fn2_launch_batch_init( s.dKeys, nJobs, fn2::kRangeSlots, jobStride, s.dCounter, (int)shape.size() * fn2::kQueueCounterInts, s.stream ), "range reset" ) )
+                if( !fn2::HipOk( (hipError_t)fn2_launch_batch_init( s.dKeys, nJobs, fn2::kRangeSlots, fn2::kRangeStrideSpread, s.dCounter,
+                                                                    (int)shape.size() * fn2::kQueueCounterInts, s.stream ), "range reset" ) )
                     return false;
             }
-            else if( !fn2::HipOk( (hipError_t)fn2_launch_minmax_init( s.dKeys, nJobs, fn2::kRangeSlots, jobStride, s.stream ), "range reset" ) ) return false;
             int first = 0;
             for( size_t gi = 0; gi < shape.size(); gi++ )
             {
                 const auto& g = shape[gi];
-                const int32_t* bj = s.dBlockJob + first;
-                const uint32_t* bb = s.dBlockBase + first;
+                const int32_t* bj = blockJob + first;
+                const uint32_t* bb = blockBase + first;
                 if( kernels[gi] && mode == FN2_SERVE_PERSISTENT )
                 {
-                    const fn2::GenArgs* jobs = s.dJobs;
                     uint32_t nTiles = (uint32_t)g[1];
                     uint32_t* counter = s.dCounter + gi * fn2::kQueueCounterInts;
                     const int64_t resident = (int64_t)cus * std::max( 1, kernels[gi]->queueBlocksPerCU );
@@ -946,7 +975,6 @@ namespace
                 }
                 else if( kernels[gi] )
                 {
-                    const fn2::GenArgs* jobs = s.dJobs;
                     void* params[] = { (void*)&jobs, (void*)&bj, (void*)&bb };
                     if( !fn2::HipOk( hipModuleLaunchKernel( kernels[gi]->batch, (unsigned)g[1], 1, 1, (unsigned)g[3], 1, 1, 0, s.stream, params, nullptr ),
                                      "specialised batch launch" ) )
@@ -957,15 +985,17 @@ namespace
                     int dm = (int)( g[0] / 16 ), fm = (int)( g[0] % 16 );
                     if( mode == FN2_SERVE_PERSISTENT )
                     {
-                        if( !fn2::HipOk( (hipError_t)fn2_launch_generate_queue( s.dJobs, bj, bb, (int)g[1], dm, fm, (int)g[2], s.dCounter + gi * fn2::kQueueCounterInts, s.stream ),
+                        if( !fn2::HipOk( (hipError_t)fn2_launch_generate_queue( jobs, bj, bb, (int)g[1], dm, fm, (int)g[2], s.dCounter + gi * fn2::kQueueCounterInts, s.stream ),
                                          "work-queue launch" ) )
                             return false;
                     }
-                    else if( !fn2::HipOk( (hipError_t)fn2_launch_generate_batch( s.dJobs, bj, bb, (int)g[1], dm, fm, (int)g[2], s.stream ), "batch launch" ) )
+                    else if( !fn2::HipOk( (hipError_t)fn2_launch_generate_batch( jobs, bj, bb, (int)g[1], dm, fm, (int)g[2], s.stream ), "batch launch" ) )
                         return false;
                 }
                 first += (int)g[1];
             }
+            if( mode != FN2_SERVE_PERSISTENT && !s.rangeDirect )
+                return fn2::HipOk( (hipError_t)fn2_launch_range_reduce( jobs, {}, nJobs, s.hRange, s.stream ), "range reduction" );
             return true;
         }
 
@@ -985,7 +1015,8 @@ namespace
                     return false;
             }
             if( stagedEnd && !fn2::HipOk( hipMemcpyAsync( s.hOut, s.dOut, stagedEnd * 4, hipMemcpyDeviceToHost, s.stream ), "copy outputs" ) ) return false;
-            if( !fn2::HipOk( hipMemcpyAsync( s.hKeys, s.dKeys, jobRangeInts * sizeof( int32_t ) * nJobs, hipMemcpyDeviceToHost, s.stream ), "copy ranges" ) ) return false;
+            if( mode == FN2_SERVE_PERSISTENT &&
+                !fn2::HipOk( hipMemcpyAsync( s.hKeys, s.dKeys, jobRangeInts * sizeof( int32_t ) * nJobs, hipMemcpyDeviceToHost, s.stream ), "copy ranges" ) ) return false;
             // the work-queue counters: how many pulls each launch made
             if( s.queueLaunches &&
                 !fn2::HipOk( hipMemcpyAsync( s.hKeys + (size_t)jobRangeInts * kMaxJobs, s.dCounter,
@@ -1049,7 +1080,12 @@ namespace
                     copies->Run( segs );
                     for( Request* r : s.reqs )
                     {
-                        if( !fn2::DecodeRange( s.hKeys + (size_t)r->job * jobRangeInts, fn2::kRangeSlots, jobStride, r->mm[0], r->mm[1] ) )
+                        const bool any = mode == FN2_SERVE_PERSISTENT
+                            ? fn2::DecodeRange( s.hKeys + (size_t)r->job * jobRangeInts, fn2::kRangeSlots, fn2::kRangeStrideSpread, r->mm[0], r->mm[1] )
+                            : s.rangeDirect
+                            ? fn2::DecodeRange( s.hRange + (size_t)2 * r->firstBlock, r->blocks, 2, r->mm[0], r->mm[1] )
+                            : fn2::DecodeRange( s.hRange + (size_t)2 * r->job, 1, 2, r->mm[0], r->mm[1] );
+                        if( !any )
                         {
                             r->mm[0] = __builtin_inff();
                             r->mm[1] = -__builtin_inff();
