@@ -1075,7 +1075,7 @@ namespace fn2d
         v[1] = fmadd( m, fmsub( f[1], gX, f[0] * gY ), v[1] );
     }
     // Orthogonal gradient matrix, 3D (:237-316, generic branch)
-    FN2D void orthoVec3( int32_t h31, const float* f, float m, float* v )
+    FN2D void orthoSelect3( int32_t h31, const float* f, float m, float* v )
     {
         const float kA = 2.224744871391589f, kB = -0.224744871391589f, kC = -1.0f, kDE = 1.0f, kF = 2.0f;
         int32_t hs = isrl( h31, 1 );
@@ -1104,6 +1104,68 @@ namespace fn2d
         v[1] = fmadd( m, ip3 == 1 ? valueC : ( ip3 == 2 ? valueBA : valueAB ), v[1] );
         v[2] = fmadd( m, ip3 == 2 ? valueC : valueBA, v[2] );
     }
+#if defined( __HIP_DEVICE_COMPILE__ )
+    // orthoVec3's matrices as a table in LDS: the three rows that the hash
+    // bits it looks at choose, for each of their 128 combinations. On MI355X
+    // the generic branch costs about 190 cycles of a SIMD per wave and vertex,
+    // nearly all of them choosing the rows; finding the entry and turning the
+    // offset by it about 70 (see gradDot3's table). The products and sums are
+    // the same.
+    struct alignas( 16 ) OrthoEntry
+    {
+        float r[3][4];
+    };
+    constexpr int kOrthoEntries = 128;
+    __device__ __forceinline__ OrthoEntry* orthoTable3()
+    {
+        __shared__ OrthoEntry t[kOrthoEntries];
+        return t;
+    }
+    // ifb: bits 0-1 the signs, 2 which value comes first, 30-31 the axis left out; ip3: 0..3
+    __device__ __forceinline__ int orthoIndex( int32_t ifb, int32_t ip3 ) { return ( ifb & 7 ) | ( isrl( ifb, 30 ) << 3 ) | ( ip3 << 5 ); }
+    __device__ __forceinline__ void fillOrthoTable3( int e )
+    {
+        if( e >= kOrthoEntries ) return;
+        const float kA = 2.224744871391589f, kB = -0.224744871391589f, kC = -1.0f, kDE = 1.0f, kF = 2.0f;
+        const int32_t s0 = ishl( e, 31 ), s1 = ishl( e >> 1, 31 );
+        const bool ba = ( e & 4 ) != 0, notXY = ( e & 8 ) != 0, notYZ = ( e & 16 ) != 0;
+        const int ip3 = e >> 5;
+        // a row: p on the first axis that is not left out, q on the second,
+        // c on the one left out
+        auto row = [&]( float* r, float p, float q, float c ) {
+            p = fxor( p, s0 );
+            q = fxor( q, s1 );
+            r[0] = notYZ ? c : p;
+            r[1] = notXY ? q : notYZ ? p : c;
+            r[2] = notXY ? c : q;
+            r[3] = 0.0f;
+        };
+        const float first = ba ? kB : kA, second = ba ? kA : kB;
+        OrthoEntry t;
+        float rc[4], rab[4], rba[4];
+        row( rc, kDE, kDE, kF );
+        row( rab, first, second, kC );
+        row( rba, second, first, kC );
+#pragma unroll
+        for( int a = 0; a < 4; a++ )
+        {
+            t.r[0][a] = ip3 == 0 ? rc[a] : rab[a];
+            t.r[1][a] = ip3 == 1 ? rc[a] : ip3 == 2 ? rba[a] : rab[a];
+            t.r[2][a] = ip3 == 2 ? rc[a] : rba[a];
+        }
+        orthoTable3()[e] = t;
+    }
+    __device__ __forceinline__ void orthoVec3( int32_t h31, const float* f, float m, float* v )
+    {
+        const int32_t hs = isrl( h31, 1 );
+        const OrthoEntry& e = orthoTable3()[orthoIndex( imul( hs, (int32_t)0xAAAAAAABu ), isrl( imul( hs, 3 ), 30 ) )];
+        m = fxor( m, ishl( h31, 31 ) );
+#pragma unroll
+        for( int a = 0; a < 3; a++ ) v[a] = fmadd( m, fmadd( e.r[a][2], f[2], fmadd( f[1], e.r[a][1], f[0] * e.r[a][0] ) ), v[a] );
+    }
+#else
+    FN2D void orthoVec3( int32_t h31, const float* f, float m, float* v ) { orthoSelect3( h31, f, m, v ); }
+#endif
     // Orthogonal gradient matrix, 4D (:318-694, generic branch)
     FN2D void orthoVec4( int32_t h31, const float* f, float m, float* v )
     {

@@ -27,11 +27,6 @@
 #ifndef FN2_UNIFORM_WARP
 #define FN2_UNIFORM_WARP 1
 #endif
-// Specialised fused fractals try the wave-uniform lattice cell of their
-// leaf (simplex2<G, true>); defined 0, they take the per-lane path only
-#ifndef FN2_UNIFORM_LATTICE
-#define FN2_UNIFORM_LATTICE 1
-#endif
 #ifndef FN2_CELL_TABLE
 #define FN2_CELL_TABLE 1
 #endif
@@ -80,7 +75,7 @@ namespace fn2i
     // Lattice noise on explicit coordinates; LEAF as OP above. G = false
     // leaves out the out-of-range select of the float -> int conversions, for
     // coordinates shown to lie below kUnguardedCoord in magnitude.
-    template<int D, int LEAF = -1, bool G = true, bool U = false>
+    template<int D, int LEAF = -1, bool G = true>
     FN2D float leafRaw( int op, int32_t seed, const float* x )
     {
         if constexpr( opIn<LEAF, fn2::OP_PERLIN>() )
@@ -100,7 +95,7 @@ namespace fn2i
         if constexpr( opIn<LEAF, fn2::OP_SIMPLEX>() )
             if( LEAF >= 0 || op == fn2::OP_SIMPLEX )
             {
-                if constexpr( D == 2 ) return simplex2<G, U>( seed, x[0], x[1] );
+                if constexpr( D == 2 ) return simplex2<G>( seed, x[0], x[1] );
                 else if constexpr( D == 3 ) return simplex3<G>( seed, x[0], x[1], x[2] );
                 else return simplex4<G>( seed, x[0], x[1], x[2], x[3] );
             }
@@ -128,7 +123,7 @@ namespace fn2i
     // A specialised kernel knows the octave count; FN2_OCTAVE_UNROLL (0: the
     // compiler's choice) sets how far the loop is unrolled, a per-tree tuning
     // knob of the serving engine.
-    template<int D, int LEAF, bool G, bool BRICK>
+    template<int D, int LEAF, bool G>
     FN2D float fractalOctaves( const Ins& in, const float* K, int32_t seed, const float* start )
     {
         const int leaf = in.p[0], octaves = in.p[1];
@@ -142,10 +137,7 @@ namespace fn2i
             float x[D];
 #pragma unroll
             for( int a = 0; a < D; a++ ) x[a] = pos[a] * freq;
-            // specialised kernels walking grid bricks try the wave-uniform
-            // lattice cell (rows of 64 rarely share one, and then pay the
-            // check for nothing)
-            return scaleOutput( leafRaw<D, LEAF, G, BRICK && ( LEAF >= 0 ) && FN2_UNIFORM_LATTICE>( leaf, s, x ), nMin, oScale, rMin );
+            return scaleOutput( leafRaw<D, LEAF, G>( leaf, s, x ), nMin, oScale, rMin );
         };
         float amp = 1.0f;
         float noise = octave( seed );
@@ -184,7 +176,7 @@ namespace fn2i
     // far below 2^31, where the float -> int conversion needs no select
     constexpr float kUnguardedCoord = 268435456.0f;   // 2^28
 
-    template<int D, int LEAF = -1, bool BRICK = false, class RF = const float*>
+    template<int D, int LEAF = -1, class RF = const float*>
     FN2D float fractalLeaf( const Ins& in, const float* K, int32_t seed, RF R, int p )
     {
         float pos[D];
@@ -205,9 +197,9 @@ namespace fn2i
             bool small = true;
 #pragma unroll
             for( int a = 0; a < D; a++ ) small = small && fabs_( pos[a] ) < limit;
-            if( waveAll( small ) ) return fractalOctaves<D, LEAF, false, BRICK>( in, K, seed, pos );
+            if( waveAll( small ) ) return fractalOctaves<D, LEAF, false>( in, K, seed, pos );
         }
-        return fractalOctaves<D, LEAF, true, BRICK>( in, K, seed, pos );
+        return fractalOctaves<D, LEAF, true>( in, K, seed, pos );
     }
 
     // SLOTS: distance slots CellularDistance keeps (4, or fewer when the
@@ -311,9 +303,7 @@ namespace fn2i
     // instruction's op and, for OP_FRACTAL_LEAF, its leaf op, for
     // OP_CELL_DISTANCE the number of distance slots it reads, so that only
     // the code the instruction runs is instantiated.
-    // BRICK: the point is one lane of a wave-sized grid brick (specialised
-    // kernels walking a grid in bricks)
-    template<int DM, int FT, int OP = -1, int AUX = -1, bool BRICK = false, class RF = float*>
+    template<int DM, int FT, int OP = -1, int AUX = -1, class RF = float*>
     FN2D void execIns( const Ins& in, const float* K, const int32_t seed, RF R )
     {
         {
@@ -334,9 +324,9 @@ namespace fn2i
                 if constexpr( opIn<OP, fn2::OP_FRACTAL_LEAF>() )
                 {
                     float v = 0.0f;
-                    if( ( DM & 4 ) && d == 2 ) v = fractalLeaf<2, AUX, BRICK>( in, K, seed, R, in.r[1] );
-                    else if( ( DM & 8 ) && d == 3 ) v = fractalLeaf<3, AUX, BRICK>( in, K, seed, R, in.r[1] );
-                    else if( DM & 16 ) v = fractalLeaf<4, AUX, BRICK>( in, K, seed, R, in.r[1] );
+                    if( ( DM & 4 ) && d == 2 ) v = fractalLeaf<2, AUX>( in, K, seed, R, in.r[1] );
+                    else if( ( DM & 8 ) && d == 3 ) v = fractalLeaf<3, AUX>( in, K, seed, R, in.r[1] );
+                    else if( DM & 16 ) v = fractalLeaf<4, AUX>( in, K, seed, R, in.r[1] );
                     R[in.r[0]] = v;
                 }
                 break;

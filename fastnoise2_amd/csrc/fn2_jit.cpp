@@ -113,16 +113,18 @@ namespace fn2
             return false;
         }
 
-        // a fused 2D Simplex fractal, whose octaves share their lattice cell
-        // across a wave more often in 8 x 8 bricks than in rows of 64: with
-        // the wave-uniform cell path, bricks took FBm(Simplex) 4096^2 from
-        // 0.1640 to 0.1575 ms on MI355X (bricks alone 0.1655, the uniform
-        // path on rows 0.1695)
-        bool UniformSimplex2D( const DeviceProgram& p )
+        // The LDS tables (kTable*) the program's instructions read
+        int Tables( const DeviceProgram& p )
         {
+            int t = 0;
             for( const Ins& in : p.ins )
-                if( in.op == OP_FRACTAL_LEAF && in.dim == 2 && in.p[0] == OP_SIMPLEX ) return true;
-            return false;
+            {
+                const int grad = in.dim == 2 ? kTableGrad2 : in.dim == 3 ? kTableGrad3 : kTableGrad4;
+                const int leaf = in.op == OP_FRACTAL_LEAF ? in.p[0] : in.op;
+                if( leaf == OP_PERLIN || leaf == OP_SIMPLEX || leaf == OP_SUPERSIMPLEX ) t |= grad;
+                if( ( in.op == OP_WARP_SIMPLEX || in.op == OP_WARP_SUPERSIMPLEX ) && in.dim == 3 && in.p[0] != 1 ) t |= kTableOrtho3;
+            }
+            return t;
         }
 
         // Each instruction becomes an `execIns` instantiated for its own op,
@@ -135,7 +137,7 @@ namespace fn2
             if( variant & kJitSharedWalk ) s << "#define FN2_SHARED_CELL_WALK 1\n";
             // long programs leave out the code that is duplicated per
             // instruction for coherent waves (cell tables, wave-uniform warp
-            // cells, a brick-specific program copy): measured with hipcc at
+            // cells): measured with hipcc at
             // -O3, the 355-instruction mixed tree compiled in 73 s without
             // them and 210 s with them, which a serving engine's first
             // requests would wait out on the interpreter
@@ -146,10 +148,9 @@ namespace fn2
                  "namespace {\nstruct Prog {\n"
                  "static constexpr bool kFresh = true;\n"
                  "static constexpr int kDims = " << p.dims << ";\n"
-                 "static constexpr bool kBricks = " << ( PrunedCellular( p ) || UniformSimplex2D( p ) ? "true" : "false" ) << ";\n"
-                 "static constexpr bool kBrickAware = " << ( lean ? "false" : "true" ) << ";\n"
-                 "template<bool BRICK = false>\n"
-                 "__device__ __forceinline__ float eval( const fn2::GenArgs& a, float* R ) const {\n";
+                 "static constexpr bool kBricks = " << ( PrunedCellular( p ) ? "true" : "false" ) << ";\n"
+                 "static constexpr int kTables = " << Tables( p ) << ";\n"
+                 "__device__ __forceinline__ float operator()( const fn2::GenArgs& a, float* R ) const {\n";
             // long programs get a register fence between instructions: measured
             // on MI355X, a 355-instruction tree needs 256 VGPRs without (one wave
             // per SIMD, 2.46 ms on 128^3) and 92 with (5 waves, 1.63 ms); a
@@ -175,10 +176,9 @@ namespace fn2
                 }
                 s << "  execIns<" << ( in.dim >= 2 && in.dim <= 4 ? 1 << in.dim : 4 ) << ", " << OpFeature( in.op ) << ", "
                   << (int)in.op << ", " << Aux( in )
-                  << ", BRICK>( in, k, iadd( a.seed, (int32_t)" << (uint32_t)in.seed << "u ), R ); }\n";
+                  << ">( in, k, iadd( a.seed, (int32_t)" << (uint32_t)in.seed << "u ), R ); }\n";
             }
             s << "return R[" << p.resultReg << "];\n}\n"
-                 "__device__ __forceinline__ float operator()( const fn2::GenArgs& a, float* R ) const { return eval<false>( a, R ); }\n"
                  "};\n}\n"
                  "extern \"C\" __global__ void __launch_bounds__( 256 ) fn2_jit_single( fn2::GenArgs a )\n"
                  "{ fn2k::generateSingle<256>( a, Prog() ); }\n"

@@ -100,6 +100,28 @@ namespace fn2k
         return StridedRegs<BLOCK>{ fn2RegisterFile + threadIdx.x };
     }
 
+    // Fills the lookup tables in LDS that the program reads (Prog::kTables, of
+    // fn2::kTable* bits), before the block's first point
+    template<class Prog>
+    __device__ __forceinline__ void fillTables()
+    {
+#if defined( __HIP_DEVICE_COMPILE__ )
+        constexpr int T = Prog::kTables;
+        if constexpr( T != 0 )
+        {
+            for( int e = (int)threadIdx.x; e < fn2d::kOrthoEntries; e += (int)blockDim.x )
+            {
+                if constexpr( ( T & fn2::kTableGrad2 ) != 0 ) fillGradTable2( e );
+                if constexpr( ( T & fn2::kTableGrad3 ) != 0 ) fillGradTable3( e );
+                if constexpr( ( T & fn2::kTableGrad4 ) != 0 ) fillGradTable4( e );
+                if constexpr( ( T & fn2::kTableOrtho3 ) != 0 ) fillOrthoTable3( e );
+                else break;   // the gradient tables have fewer entries than a block has threads
+            }
+            __syncthreads();
+        }
+#endif
+    }
+
     // A grid request walked in wave-sized bricks (8 x 8 in 2D, 4 x 4 x 4 in
     // 3D) instead of runs of 64 along x: the lanes of a wave then sit close
     // together in every axis, so they agree more often on which cells a pruned
@@ -129,11 +151,7 @@ namespace fn2k
                 fresh.R[0] = fmadd( (float)(int32_t)x, a.step[0], a.offset[0] );
                 fresh.R[1] = fmadd( (float)(int32_t)y, a.step[1], a.offset[1] );
                 if constexpr( D == 3 ) fresh.R[2] = fmadd( (float)(int32_t)z, a.step[2], a.offset[2] );
-                // the program knows it runs in bricks (fn2i::fractalLeaf),
-                // unless it is one copy for both walks (long programs)
-                float v;
-                if constexpr( Prog::kBrickAware ) v = prog.template eval<true>( a, fresh.R );
-                else v = prog( a, fresh.R );
+                const float v = prog( a, fresh.R );
                 // a plain store: a wave writes 16-byte pieces of 16 lines
                 // here, which the L2 merges with its neighbours' pieces;
                 // streaming stores went out piece by piece (2.8 times the
@@ -152,6 +170,7 @@ namespace fn2k
     template<int BLOCK, class Prog>
     __device__ __forceinline__ void generateSingle( const fn2::GenArgs& a, Prog prog )
     {
+        fillTables<Prog>();
         float mn = __builtin_inff(), mx = -__builtin_inff();
         auto emit = [&]( uint32_t i, float v ) {
             storeOut( a.out + i, v );
@@ -204,6 +223,7 @@ namespace fn2k
     template<int BLOCK, class Prog>
     __device__ __forceinline__ void generateTile( const fn2::GenArgs& a, uint32_t first, Prog prog )
     {
+        fillTables<Prog>();
         float mn = __builtin_inff(), mx = -__builtin_inff();
         auto emit = [&]( uint32_t i, float v ) {
             storeOut( a.out + i, v );
@@ -299,11 +319,13 @@ namespace fn2k
     // back edge: all lanes take part in the pull (lane 0 adds one, the
     // others zero) and in publishing a range. The counters only grow, so
     // every wave leaves after at most a part's items + 1 pulls and no wave
-    // waits for another.
+    // waits for another (the one barrier, after the tables are filled, comes
+    // before the loop).
     template<int BLOCK, class Prog>
     __device__ __forceinline__ void generateQueue( const fn2::GenArgs* __restrict__ jobs, const int32_t* __restrict__ tileJob,
                                                    const uint32_t* __restrict__ tileBase, uint32_t nTiles, uint32_t* counter, Prog prog )
     {
+        fillTables<Prog>();
         constexpr uint32_t kWaves = BLOCK / 64;
         const uint32_t lane = threadIdx.x & 63;
         const uint32_t items = nTiles * kWaves;

@@ -29,6 +29,8 @@ struct Interpreted
     static constexpr bool kFresh = false;   // indexes the register file at run time (kept in LDS)
     static constexpr int kDims = 0;         // a.dims at run time
     static constexpr bool kBricks = false;  // row-major walk
+    static constexpr int kTables = ( DM & 4 ? fn2::kTableGrad2 : 0 ) | ( DM & 8 ? fn2::kTableGrad3 : 0 ) | ( DM & 16 ? fn2::kTableGrad4 : 0 ) |
+                                   ( ( DM & 8 ) != 0 && ( FT & fn2::kFeatWarp ) != 0 ? fn2::kTableOrtho3 : 0 );
     template<class RF>
     __device__ __forceinline__ float operator()( const fn2::GenArgs& g, RF R ) const { return runProgram<DM, FT>( g, R ); }
 };

@@ -123,4 +123,8 @@ namespace fn2
     static constexpr int kFeatCell = 1;   // cellular ops
     static constexpr int kFeatWarp = 2;   // domain warps
     static constexpr int kFeatMisc = 4;   // white, checkerboard, sine wave, distance
+
+    // Lookup tables in LDS that a program's kernel fills (fn2_device_math.h,
+    // fn2_device_cellwarp.h)
+    static constexpr int kTableGrad2 = 1, kTableGrad3 = 2, kTableGrad4 = 4, kTableOrtho3 = 8;
 }
