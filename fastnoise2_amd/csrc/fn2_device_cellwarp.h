@@ -1114,6 +1114,7 @@ namespace fn2d
     struct alignas( 16 ) OrthoEntry
     {
         float r[3][4];
+        float pad[4];   // 64 bytes, so that the offset is shifts and masks
     };
     constexpr int kOrthoEntries = 128;
     __device__ __forceinline__ OrthoEntry* orthoTable3()
@@ -1121,8 +1122,13 @@ namespace fn2d
         __shared__ OrthoEntry t[kOrthoEntries];
         return t;
     }
-    // ifb: bits 0-1 the signs, 2 which value comes first, 30-31 the axis left out; ip3: 0..3
-    __device__ __forceinline__ int orthoIndex( int32_t ifb, int32_t ip3 ) { return ( ifb & 7 ) | ( isrl( ifb, 30 ) << 3 ) | ( ip3 << 5 ); }
+    // The byte offset of an entry: ifb's bits 0-1 (the signs), 2 (which value
+    // comes first) and 30-31 (the axis left out), then bits 30-31 of three
+    // times the hash
+    __device__ __forceinline__ int32_t orthoOffset( int32_t ifb, int32_t three )
+    {
+        return ( ishl( ifb, 6 ) & 0x1c0 ) | ( isrl( ifb, 21 ) & 0x600 ) | ( isrl( three, 19 ) & 0x1800 );
+    }
     __device__ __forceinline__ void fillOrthoTable3( int e )
     {
         if( e >= kOrthoEntries ) return;
@@ -1141,7 +1147,7 @@ namespace fn2d
             r[3] = 0.0f;
         };
         const float first = ba ? kB : kA, second = ba ? kA : kB;
-        OrthoEntry t;
+        OrthoEntry t{};
         float rc[4], rab[4], rba[4];
         row( rc, kDE, kDE, kF );
         row( rab, first, second, kC );
@@ -1158,7 +1164,8 @@ namespace fn2d
     __device__ __forceinline__ void orthoVec3( int32_t h31, const float* f, float m, float* v )
     {
         const int32_t hs = isrl( h31, 1 );
-        const OrthoEntry& e = orthoTable3()[orthoIndex( imul( hs, (int32_t)0xAAAAAAABu ), isrl( imul( hs, 3 ), 30 ) )];
+        const int32_t offset = orthoOffset( imul( hs, (int32_t)0xAAAAAAABu ), iadd( iadd( hs, hs ), hs ) );
+        const OrthoEntry& e = *reinterpret_cast<const OrthoEntry*>( reinterpret_cast<const char*>( orthoTable3() ) + offset );
         m = fxor( m, ishl( h31, 31 ) );
 #pragma unroll
         for( int a = 0; a < 3; a++ ) v[a] = fmadd( m, fmadd( e.r[a][2], f[2], fmadd( f[1], e.r[a][1], f[0] * e.r[a][0] ) ), v[a] );
@@ -1327,25 +1334,26 @@ namespace fn2d
     {
         constexpr double kSkew2 = 1.0 / ( kRoot3 + 1.0 );
         constexpr double kUnskew2 = -1.0 / ( kRoot3 + 3.0 );
+        seed = inVector( seed );
         float x = sp[0], y = sp[1];
         float skewDelta = (float)kSkew2 * ( x + y );
         float xSk = x + skewDelta, ySk = y + skewDelta;
         float xB = ffloor( xSk ), yB = ffloor( ySk );
         float dxS = xSk - xB, dyS = ySk - yB;
         int32_t xP = imul( floorToInt( xB ), kPX ), yP = imul( floorToInt( yB ), kPY );
-        bool xGEy = dxS >= dyS;
+        const int32_t yAbove = lessMask( dxS, dyS );
         float unskewDelta = (float)kUnskew2 * ( dxS + dyS );
         float d0[2] = { dxS + unskewDelta, dyS + unskewDelta };
-        float d1[2] = { ( xGEy ? d0[0] : d0[0] + 1.0f ) - (float)( kUnskew2 + 1 ), ( xGEy ? d0[1] + 1.0f : d0[1] ) - (float)( kUnskew2 + 1 ) };
+        float d1[2] = { ( d0[0] + maskedOne( yAbove ) ) - (float)( kUnskew2 + 1 ), ( d0[1] + maskedOne( ~yAbove ) ) - (float)( kUnskew2 + 1 ) };
         float d2[2] = { d0[0] - (float)( kUnskew2 * 2 + 1 ), d0[1] - (float)( kUnskew2 * 2 + 1 ) };
         float f0 = fnmadd( d0[0], d0[0], fnmadd( d0[1], d0[1], 0.5f ) );
         float f1 = fnmadd( d1[0], d1[0], fnmadd( d1[1], d1[1], 0.5f ) );
         float f2 = f0 + fmadd( unskewDelta, (float)( -4.0 * ( kRoot3 + 2.0 ) / ( kRoot3 + 3.0 ) ), (float)( -2.0 / 3.0 ) );
-        f0 = fmaxf_( f0, 0.0f ); f1 = fmaxf_( f1, 0.0f ); f2 = fmaxf_( f2, 0.0f );
+        f0 = clampPositive( f0 ); f1 = clampPositive( f1 ); f2 = clampPositive( f2 );
         f0 *= f0; f0 *= f0; f1 *= f1; f1 *= f1; f2 *= f2; f2 *= f2;
         float v[2] = { 0.0f, 0.0f };
         vecContribution<2>( scheme, hash2( seed, xP, yP ), d0, f0, v );
-        vecContribution<2>( scheme, hash2( seed, xGEy ? iadd( xP, kPX ) : xP, xGEy ? yP : iadd( yP, kPY ) ), d1, f1, v );
+        vecContribution<2>( scheme, hash2( seed, bitSelect( yAbove, xP, iadd( xP, kPX ) ), bitSelect( yAbove, iadd( yP, kPY ), yP ) ), d1, f1, v );
         vecContribution<2>( scheme, hash2( seed, iadd( xP, kPX ), iadd( yP, kPY ) ), d2, f2, v );
         const float kBound = scheme == 1 ? (float)( 49.918426513671875 / 2.0 ) : 70.1480577066486f;
         v[0] = v[0] * ( kBound * axisScale[0] );
@@ -1357,33 +1365,36 @@ namespace fn2d
     template<> FN2D float warpSimplex<3>( int32_t seed, int scheme, float amp, const float* axisScale, const float* sp, float* out )
     {
         constexpr double kReflectUnskew3 = -1.0 / 2.0;
+        seed = inVector( seed );
         float x = sp[0], y = sp[1], z = sp[2];
         float skewDelta = (float)( 1.0 / 3.0 ) * ( x + y + z );
         float xSk = x + skewDelta, ySk = y + skewDelta, zSk = z + skewDelta;
         float xB = ffloor( xSk ), yB = ffloor( ySk ), zB = ffloor( zSk );
         float dxS = xSk - xB, dyS = ySk - yB, dzS = zSk - zB;
         int32_t xP = imul( floorToInt( xB ), kPX ), yP = imul( floorToInt( yB ), kPY ), zP = imul( floorToInt( zB ), kPZ );
-        bool xGEy = dxS >= dyS, yGEz = dyS >= dzS, xGEz = dxS >= dzS;
+        // the axes' order as masks, as in simplex3
+        const int32_t xy = lessMask( dxS, dyS ), yz = lessMask( dyS, dzS ), xz = lessMask( dxS, dzS );
         float unskewDelta = (float)kReflectUnskew3 * ( dxS + dyS + dzS );
         float d0[3] = { dxS + unskewDelta, dyS + unskewDelta, dzS + unskewDelta };
-        bool x1m = xGEy && xGEz, y1m = yGEz && !xGEy, z1inv = xGEz || yGEz;
-        bool x2inv = xGEy || xGEz, y2m = xGEy && !yGEz, z2m = xGEz && yGEz;
+        const int32_t x1m = ~( xy | xz ), y1m = xy & ~yz, z1m = xz & yz;
+        const int32_t x2n = xy & xz, y2n = yz & ~xy, z2n = ~( xz | yz );
         const float k3 = (float)( kReflectUnskew3 * 3 + 1 );
         float d3[3] = { d0[0] - k3, d0[1] - k3, d0[2] - k3 };
-        float d1[3] = { x1m ? d3[0] - 1.0f : d3[0], y1m ? d3[1] - 1.0f : d3[1], z1inv ? d3[2] : d3[2] - 1.0f };
-        float d2[3] = { x2inv ? d0[0] : d0[0] + 1.0f, y2m ? d0[1] + 1.0f : d0[1], z2m ? d0[2] + 1.0f : d0[2] };
+        float d1[3] = { d3[0] - maskedOne( x1m ), d3[1] - maskedOne( y1m ), d3[2] - maskedOne( z1m ) };
+        float d2[3] = { d0[0] + maskedOne( x2n ), d0[1] + maskedOne( y2n ), d0[2] + maskedOne( z2n ) };
         const float fr = (float)0.6;
         float f0 = fnmadd( d0[2], d0[2], fnmadd( d0[1], d0[1], fnmadd( d0[0], d0[0], fr ) ) );
         float f1 = fnmadd( d1[2], d1[2], fnmadd( d1[1], d1[1], fnmadd( d1[0], d1[0], fr ) ) );
         float f2 = fnmadd( d2[2], d2[2], fnmadd( d2[1], d2[1], fnmadd( d2[0], d2[0], fr ) ) );
         float f3 = f0 - ( unskewDelta + (float)( 3.0 / 4.0 ) );
-        f0 = fmaxf_( f0, 0.0f ); f1 = fmaxf_( f1, 0.0f ); f2 = fmaxf_( f2, 0.0f ); f3 = fmaxf_( f3, 0.0f );
+        f0 = clampPositive( f0 ); f1 = clampPositive( f1 ); f2 = clampPositive( f2 ); f3 = clampPositive( f3 );
         f0 *= f0; f0 *= f0; f1 *= f1; f1 *= f1; f2 *= f2; f2 *= f2; f3 *= f3; f3 *= f3;
         float v[3] = { 0.0f, 0.0f, 0.0f };
+        const int32_t x1 = iadd( xP, kPX ), y1 = iadd( yP, kPY ), z1 = iadd( zP, kPZ );
         vecContribution<3>( scheme, hash3( seed, xP, yP, zP ), d0, f0, v );
-        vecContribution<3>( scheme, hash3( seed, x1m ? iadd( xP, kPX ) : xP, y1m ? iadd( yP, kPY ) : yP, z1inv ? zP : iadd( zP, kPZ ) ), d1, f1, v );
-        vecContribution<3>( scheme, hash3( seed, x2inv ? iadd( xP, kPX ) : xP, y2m ? yP : iadd( yP, kPY ), z2m ? zP : iadd( zP, kPZ ) ), d2, f2, v );
-        vecContribution<3>( scheme, hash3( seed, iadd( xP, kPX ), iadd( yP, kPY ), iadd( zP, kPZ ) ), d3, f3, v );
+        vecContribution<3>( scheme, hash3( seed, bitSelect( x1m, x1, xP ), bitSelect( y1m, y1, yP ), bitSelect( z1m, z1, zP ) ), d1, f1, v );
+        vecContribution<3>( scheme, hash3( seed, bitSelect( x2n, xP, x1 ), bitSelect( y2n, yP, y1 ), bitSelect( z2n, zP, z1 ) ), d2, f2, v );
+        vecContribution<3>( scheme, hash3( seed, x1, y1, z1 ), d3, f3, v );
         if( scheme == 1 )
         {
             float delta = (float)( -2.0 / 2.0 ) * ( v[0] + v[1] + v[2] );
@@ -1405,20 +1416,23 @@ namespace fn2d
         const int32_t prime[4] = { kPX, kPY, kPZ, kPW };
         float unskewDelta = (float)kUnskew4 * ( dxS + dyS + dzS + dwS );
         float d0[4] = { dxS + unskewDelta, dyS + unskewDelta, dzS + unskewDelta, dwS + unskewDelta };
-        int rank[4] = { 0, 0, 0, 0 };
+        // as in simplex4
+        int32_t rank[4] = { 3, 2, 1, 0 };
 #pragma unroll
         for( int a = 0; a < 4; a++ )
 #pragma unroll
             for( int b = a + 1; b < 4; b++ )
             {
-                if( d0[a] >= d0[b] ) rank[a]++; else rank[b]++;
+                const int32_t less = lessMask( d0[a], d0[b] );
+                rank[a] = iadd( rank[a], less );
+                rank[b] = isub( rank[b], less );
             }
         const float fr = (float)0.6;
         float v[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
         float f0 = fnmadd( d0[3], d0[3], fnmadd( d0[2], d0[2], fnmadd( d0[1], d0[1], fnmadd( d0[0], d0[0], fr ) ) ) );
         float f4 = f0 + fmadd( unskewDelta, (float)( -4.0 * ( kRoot5 + 3.0 ) / ( kRoot5 + 5.0 ) ), (float)( -4.0 / 5.0 ) );
         {
-            float f = fmaxf_( f0, 0.0f ); f *= f; f *= f;
+            float f = clampPositive( f0 ); f *= f; f *= f;
             vecContribution<4>( scheme, hash4( seed, base[0], base[1], base[2], base[3] ), d0, f, v );
         }
 #pragma unroll
@@ -1430,18 +1444,18 @@ namespace fn2d
 #pragma unroll
             for( int a = 0; a < 4; a++ )
             {
-                bool m = rank[a] > 3 - vi;
-                d[a] = ( m ? d0[a] - 1.0f : d0[a] ) - u;
-                hp[a] = m ? iadd( base[a], prime[a] ) : base[a];
+                const int32_t m = inVector( isub( 3 - vi, rank[a] ) ) >> 31;
+                d[a] = ( d0[a] - maskedOne( m ) ) - u;
+                hp[a] = bitSelect( m, iadd( base[a], prime[a] ), base[a] );
             }
             float f = fnmadd( d[3], d[3], fnmadd( d[2], d[2], fnmadd( d[1], d[1], fnmadd( d[0], d[0], fr ) ) ) );
-            f = fmaxf_( f, 0.0f ); f *= f; f *= f;
+            f = clampPositive( f ); f *= f; f *= f;
             vecContribution<4>( scheme, hash4( seed, hp[0], hp[1], hp[2], hp[3] ), d, f, v );
         }
         {
             const float u4 = (float)( kUnskew4 * 4 + 1 );
             float d[4] = { d0[0] - u4, d0[1] - u4, d0[2] - u4, d0[3] - u4 };
-            float f = fmaxf_( f4, 0.0f ); f *= f; f *= f;
+            float f = clampPositive( f4 ); f *= f; f *= f;
             vecContribution<4>( scheme, hash4( seed, iadd( base[0], kPX ), iadd( base[1], kPY ), iadd( base[2], kPZ ), iadd( base[3], kPW ) ), d, f, v );
         }
         const float kBound = scheme == 1 ? (float)( 33.653125584827855 / 1.4142135623730951 ) : 30.88161777516092f;
@@ -1451,13 +1465,14 @@ namespace fn2d
     // DomainWarpSuperSimplex::Warp (DomainWarpSimplex.inl:1131-1836); no seed offset
     template<int D> FN2D float warpSuperSimplex( int32_t seed, int scheme, float amp, const float* axisScale, const float* sp, float* out )
     {
+        seed = inVector( seed );
         float v[D];
 #pragma unroll
         for( int a = 0; a < D; a++ ) v[a] = 0.0f;
         auto vtx = [&]( int32_t h, const float* d, float f, bool ) { vecContribution<D>( scheme, h, d, f, v ); };
         if constexpr( D == 2 )
         {
-            superWalk2( seed, sp[0], sp[1], vtx );
+            superWalk2<true, false>( seed, sp[0], sp[1], vtx );
             const float kBound = scheme == 1 ? (float)( 9.28993664146183 / 2.0 ) : 12.814453124999995f;
             v[0] = v[0] * ( kBound * axisScale[0] );
             v[1] = v[1] * ( kBound * axisScale[1] );
@@ -1467,7 +1482,7 @@ namespace fn2d
         }
         else if constexpr( D == 3 )
         {
-            superWalk3( seed, sp[0], sp[1], sp[2], vtx );
+            superWalk3<true, false>( seed, sp[0], sp[1], sp[2], vtx );
             if( scheme == 1 )
             {
                 float delta = (float)( -2.0 / 3.0 ) * ( v[0] + v[1] + v[2] );
@@ -1478,7 +1493,7 @@ namespace fn2d
         }
         else
         {
-            superWalk4( seed, sp[0], sp[1], sp[2], sp[3], vtx );
+            superWalk4<true, false>( seed, sp[0], sp[1], sp[2], sp[3], vtx );
             const float kBound = scheme == 1 ? (float)( 115.21625311930542 / 1.4142135623730951 ) : 48.80058117543753f;
             return warpFinish<4>( kBound, axisScale, amp, v, out );
         }

@@ -23,8 +23,8 @@ namespace fn2d
         float xf0 = x - xs, yf0 = y - ys;
         float xf1 = xf0 - 1.0f, yf1 = yf0 - 1.0f;
         float xq = interpQuintic( xf0 ), yq = interpQuintic( yf0 );
-        return lerp( lerp( gradDot2( hash2( seed, x0, y0 ), xf0, yf0 ), gradDot2( hash2( seed, x1, y0 ), xf1, yf0 ), xq ),
-                     lerp( gradDot2( hash2( seed, x0, y1 ), xf0, yf1 ), gradDot2( hash2( seed, x1, y1 ), xf1, yf1 ), xq ), yq );
+        return lerp( lerp( gradDot2( gradHash2( seed, x0, y0 ), xf0, yf0 ), gradDot2( gradHash2( seed, x1, y0 ), xf1, yf0 ), xq ),
+                     lerp( gradDot2( gradHash2( seed, x0, y1 ), xf0, yf1 ), gradDot2( gradHash2( seed, x1, y1 ), xf1, yf1 ), xq ), yq );
     }
     template<bool G = true>
     FN2D float perlin3( int32_t seed, float x, float y, float z )
@@ -35,10 +35,10 @@ namespace fn2d
         float xf0 = x - xs, yf0 = y - ys, zf0 = z - zs;
         float xf1 = xf0 - 1.0f, yf1 = yf0 - 1.0f, zf1 = zf0 - 1.0f;
         float xq = interpQuintic( xf0 ), yq = interpQuintic( yf0 ), zq = interpQuintic( zf0 );
-        float l0 = lerp( lerp( gradDot3( hash3( seed, x0, y0, z0 ), xf0, yf0, zf0 ), gradDot3( hash3( seed, x1, y0, z0 ), xf1, yf0, zf0 ), xq ),
-                         lerp( gradDot3( hash3( seed, x0, y1, z0 ), xf0, yf1, zf0 ), gradDot3( hash3( seed, x1, y1, z0 ), xf1, yf1, zf0 ), xq ), yq );
-        float l1 = lerp( lerp( gradDot3( hash3( seed, x0, y0, z1 ), xf0, yf0, zf1 ), gradDot3( hash3( seed, x1, y0, z1 ), xf1, yf0, zf1 ), xq ),
-                         lerp( gradDot3( hash3( seed, x0, y1, z1 ), xf0, yf1, zf1 ), gradDot3( hash3( seed, x1, y1, z1 ), xf1, yf1, zf1 ), xq ), yq );
+        float l0 = lerp( lerp( gradDot3( gradHash3( seed, x0, y0, z0 ), xf0, yf0, zf0 ), gradDot3( gradHash3( seed, x1, y0, z0 ), xf1, yf0, zf0 ), xq ),
+                         lerp( gradDot3( gradHash3( seed, x0, y1, z0 ), xf0, yf1, zf0 ), gradDot3( gradHash3( seed, x1, y1, z0 ), xf1, yf1, zf0 ), xq ), yq );
+        float l1 = lerp( lerp( gradDot3( gradHash3( seed, x0, y0, z1 ), xf0, yf0, zf1 ), gradDot3( gradHash3( seed, x1, y0, z1 ), xf1, yf0, zf1 ), xq ),
+                         lerp( gradDot3( gradHash3( seed, x0, y1, z1 ), xf0, yf1, zf1 ), gradDot3( gradHash3( seed, x1, y1, z1 ), xf1, yf1, zf1 ), xq ), yq );
         return lerp( l0, l1, zq );
     }
     template<bool G = true>
@@ -62,8 +62,8 @@ namespace fn2d
             {
                 int32_t zp = zi ? z1 : z0;
                 float zf = zi ? zf1 : zf0;
-                zl[zi] = lerp( lerp( gradDot4( hash4( seed, x0, y0, zp, wp ), xf0, yf0, zf, wf ), gradDot4( hash4( seed, x1, y0, zp, wp ), xf1, yf0, zf, wf ), xq ),
-                               lerp( gradDot4( hash4( seed, x0, y1, zp, wp ), xf0, yf1, zf, wf ), gradDot4( hash4( seed, x1, y1, zp, wp ), xf1, yf1, zf, wf ), xq ), yq );
+                zl[zi] = lerp( lerp( gradDot4( gradHash4( seed, x0, y0, zp, wp ), xf0, yf0, zf, wf ), gradDot4( gradHash4( seed, x1, y0, zp, wp ), xf1, yf0, zf, wf ), xq ),
+                               lerp( gradDot4( gradHash4( seed, x0, y1, zp, wp ), xf0, yf1, zf, wf ), gradDot4( gradHash4( seed, x1, y1, zp, wp ), xf1, yf1, zf, wf ), xq ), yq );
             }
             v[wi] = lerp( zl[0], zl[1], zq );
         }
@@ -132,21 +132,21 @@ namespace fn2d
         float xB = ffloor( xSk ), yB = ffloor( ySk );
         float dxS = xSk - xB, dyS = ySk - yB;
         int32_t xP = imul( floorToInt<G>( xB ), kPX ), yP = imul( floorToInt<G>( yB ), kPY );
-        bool xGEy = dxS >= dyS;
+        const int32_t yAbove = lessMask( dxS, dyS );   // the middle vertex is a step along y, else along x
         float unskewDelta = (float)kUnskew2 * ( dxS + dyS );
         float dx0 = dxS + unskewDelta, dy0 = dyS + unskewDelta;
-        float dx1 = ( xGEy ? dx0 : dx0 + 1.0f ) - (float)( kUnskew2 + 1 );
-        float dy1 = ( xGEy ? dy0 + 1.0f : dy0 ) - (float)( kUnskew2 + 1 );
+        float dx1 = ( dx0 + maskedOne( yAbove ) ) - (float)( kUnskew2 + 1 );
+        float dy1 = ( dy0 + maskedOne( ~yAbove ) ) - (float)( kUnskew2 + 1 );
         float dx2 = dx0 - (float)( kUnskew2 * 2 + 1 );
         float dy2 = dy0 - (float)( kUnskew2 * 2 + 1 );
         float f0 = fnmadd( dx0, dx0, fnmadd( dy0, dy0, 0.5f ) );
         float f1 = fnmadd( dx1, dx1, fnmadd( dy1, dy1, 0.5f ) );
         float f2 = f0 + fmadd( unskewDelta, (float)( -4.0 * ( kRoot3 + 2.0 ) / ( kRoot3 + 3.0 ) ), (float)( -2.0 / 3.0 ) );
-        f0 = fmaxf_( f0, 0.0f ); f1 = fmaxf_( f1, 0.0f ); f2 = fmaxf_( f2, 0.0f );
+        f0 = clampPositive( f0 ); f1 = clampPositive( f1 ); f2 = clampPositive( f2 );
         f0 *= f0; f0 *= f0; f1 *= f1; f1 *= f1; f2 *= f2; f2 *= f2;
-        float g0 = gradDot2( hash2( seed, xP, yP ), dx0, dy0 );
-        float g1 = gradDot2( hash2( seed, xGEy ? iadd( xP, kPX ) : xP, xGEy ? yP : iadd( yP, kPY ) ), dx1, dy1 );
-        float g2 = gradDot2( hash2( seed, iadd( xP, kPX ), iadd( yP, kPY ) ), dx2, dy2 );
+        float g0 = gradDot2( gradHash2( seed, xP, yP ), dx0, dy0 );
+        float g1 = gradDot2( gradHash2( seed, bitSelect( yAbove, xP, iadd( xP, kPX ) ), bitSelect( yAbove, iadd( yP, kPY ), yP ) ), dx1, dy1 );
+        float g2 = gradDot2( gradHash2( seed, iadd( xP, kPX ), iadd( yP, kPY ) ), dx2, dy2 );
         return fmadd( g0, f0, fmadd( g1, f1, g2 * f2 ) );
     }
     template<bool G = true>
@@ -158,31 +158,33 @@ namespace fn2d
         float xB = ffloor( xSk ), yB = ffloor( ySk ), zB = ffloor( zSk );
         float dxS = xSk - xB, dyS = ySk - yB, dzS = zSk - zB;
         int32_t xP = imul( floorToInt<G>( xB ), kPX ), yP = imul( floorToInt<G>( yB ), kPY ), zP = imul( floorToInt<G>( zB ), kPZ );
-        bool xGEy = dxS >= dyS, yGEz = dyS >= dzS, xGEz = dxS >= dzS;
+        // which of two axes is the larger, as masks (lessMask)
+        const int32_t xy = lessMask( dxS, dyS ), yz = lessMask( dyS, dzS ), xz = lessMask( dxS, dzS );
         float unskewDelta = (float)kReflectUnskew3 * ( dxS + dyS + dzS );
         float dx0 = dxS + unskewDelta, dy0 = dyS + unskewDelta, dz0 = dzS + unskewDelta;
         // vertex 1 = the largest axis; vertex 2 = all but the smallest axis
-        bool x1m = xGEy && xGEz, y1m = yGEz && !xGEy, z1inv = xGEz || yGEz;
-        bool x2inv = xGEy || xGEz, y2m = xGEy && !yGEz, z2m = xGEz && yGEz;
+        const int32_t x1m = ~( xy | xz ), y1m = xy & ~yz, z1m = xz & yz;
+        const int32_t x2n = xy & xz, y2n = yz & ~xy, z2n = ~( xz | yz );
         const float k3 = (float)( kReflectUnskew3 * 3 + 1 );
         float dx3 = dx0 - k3, dy3 = dy0 - k3, dz3 = dz0 - k3;
-        float dx1 = x1m ? dx3 - 1.0f : dx3;
-        float dy1 = y1m ? dy3 - 1.0f : dy3;
-        float dz1 = z1inv ? dz3 : dz3 - 1.0f;
-        float dx2 = x2inv ? dx0 : dx0 + 1.0f;
-        float dy2 = y2m ? dy0 + 1.0f : dy0;
-        float dz2 = z2m ? dz0 + 1.0f : dz0;
+        float dx1 = dx3 - maskedOne( x1m );
+        float dy1 = dy3 - maskedOne( y1m );
+        float dz1 = dz3 - maskedOne( z1m );
+        float dx2 = dx0 + maskedOne( x2n );
+        float dy2 = dy0 + maskedOne( y2n );
+        float dz2 = dz0 + maskedOne( z2n );
         const float fr = (float)0.6;
         float f0 = fnmadd( dz0, dz0, fnmadd( dy0, dy0, fnmadd( dx0, dx0, fr ) ) );
         float f1 = fnmadd( dz1, dz1, fnmadd( dy1, dy1, fnmadd( dx1, dx1, fr ) ) );
         float f2 = fnmadd( dz2, dz2, fnmadd( dy2, dy2, fnmadd( dx2, dx2, fr ) ) );
         float f3 = f0 - ( unskewDelta + (float)( 3.0 / 4.0 ) );
-        f0 = fmaxf_( f0, 0.0f ); f1 = fmaxf_( f1, 0.0f ); f2 = fmaxf_( f2, 0.0f ); f3 = fmaxf_( f3, 0.0f );
+        f0 = clampPositive( f0 ); f1 = clampPositive( f1 ); f2 = clampPositive( f2 ); f3 = clampPositive( f3 );
         f0 *= f0; f0 *= f0; f1 *= f1; f1 *= f1; f2 *= f2; f2 *= f2; f3 *= f3; f3 *= f3;
-        float g0 = gradDot3( hash3( seed, xP, yP, zP ), dx0, dy0, dz0 );
-        float g1 = gradDot3( hash3( seed, x1m ? iadd( xP, kPX ) : xP, y1m ? iadd( yP, kPY ) : yP, z1inv ? zP : iadd( zP, kPZ ) ), dx1, dy1, dz1 );
-        float g2 = gradDot3( hash3( seed, x2inv ? iadd( xP, kPX ) : xP, y2m ? yP : iadd( yP, kPY ), z2m ? zP : iadd( zP, kPZ ) ), dx2, dy2, dz2 );
-        float g3 = gradDot3( hash3( seed, iadd( xP, kPX ), iadd( yP, kPY ), iadd( zP, kPZ ) ), dx3, dy3, dz3 );
+        const int32_t x1 = iadd( xP, kPX ), y1 = iadd( yP, kPY ), z1 = iadd( zP, kPZ );
+        float g0 = gradDot3( gradHash3( seed, xP, yP, zP ), dx0, dy0, dz0 );
+        float g1 = gradDot3( gradHash3( seed, bitSelect( x1m, x1, xP ), bitSelect( y1m, y1, yP ), bitSelect( z1m, z1, zP ) ), dx1, dy1, dz1 );
+        float g2 = gradDot3( gradHash3( seed, bitSelect( x2n, xP, x1 ), bitSelect( y2n, yP, y1 ), bitSelect( z2n, zP, z1 ) ), dx2, dy2, dz2 );
+        float g3 = gradDot3( gradHash3( seed, x1, y1, z1 ), dx3, dy3, dz3 );
         return fmadd( g3, f3, fmadd( g2, f2, fmadd( g1, f1, g0 * f0 ) ) );
     }
     template<bool G = true>
@@ -198,13 +200,15 @@ namespace fn2d
         float unskewDelta = (float)kUnskew4 * ( dxS + dyS + dzS + dwS );
         float d0[4] = { dxS + unskewDelta, dyS + unskewDelta, dzS + unskewDelta, dwS + unskewDelta };
         // rank of each axis among the four (ties resolved by axis order)
-        int rank[4] = { 0, 0, 0, 0 };
+        int32_t rank[4] = { 3, 2, 1, 0 };
 #pragma unroll
         for( int a = 0; a < 4; a++ )
 #pragma unroll
             for( int b = a + 1; b < 4; b++ )
             {
-                if( d0[a] >= d0[b] ) rank[a]++; else rank[b]++;
+                const int32_t less = lessMask( d0[a], d0[b] );
+                rank[a] = iadd( rank[a], less );
+                rank[b] = isub( rank[b], less );
             }
         const int32_t prime[4] = { kPX, kPY, kPZ, kPW };
         const int32_t base[4] = { xP, yP, zP, wP };
@@ -214,9 +218,9 @@ namespace fn2d
         float f4 = f0 + fmadd( unskewDelta, (float)( -4.0 * ( kRoot5 + 3.0 ) / ( kRoot5 + 5.0 ) ), (float)( -4.0 / 5.0 ) );
         // vertices 4, 3, 2, 1 then 0 to reproduce FMulAdd( g0, f0, FMulAdd( g1, f1, ... g4 * f4 ) )
         {
-            float f = fmaxf_( f4, 0.0f ); f *= f; f *= f;
+            float f = clampPositive( f4 ); f *= f; f *= f;
             const float u4 = (float)( kUnskew4 * 4 + 1 );
-            float g = gradDot4( hash4( seed, iadd( xP, kPX ), iadd( yP, kPY ), iadd( zP, kPZ ), iadd( wP, kPW ) ), d0[0] - u4, d0[1] - u4, d0[2] - u4, d0[3] - u4 );
+            float g = gradDot4( gradHash4( seed, iadd( xP, kPX ), iadd( yP, kPY ), iadd( zP, kPZ ), iadd( wP, kPW ) ), d0[0] - u4, d0[1] - u4, d0[2] - u4, d0[3] - u4 );
             value = g * f;
         }
 #pragma unroll
@@ -228,26 +232,29 @@ namespace fn2d
 #pragma unroll
             for( int a = 0; a < 4; a++ )
             {
-                bool m = rank[a] > 3 - v;
-                d[a] = ( m ? d0[a] - 1.0f : d0[a] ) - u;
-                hp[a] = m ? iadd( base[a], prime[a] ) : base[a];
+                // rank above 3 - v (hidden from the compiler, which would compare and select)
+                const int32_t m = inVector( isub( 3 - v, rank[a] ) ) >> 31;
+                d[a] = ( d0[a] - maskedOne( m ) ) - u;
+                hp[a] = bitSelect( m, iadd( base[a], prime[a] ), base[a] );
             }
             float f = fnmadd( d[3], d[3], fnmadd( d[2], d[2], fnmadd( d[1], d[1], fnmadd( d[0], d[0], fr ) ) ) );
-            f = fmaxf_( f, 0.0f ); f *= f; f *= f;
-            value = fmadd( gradDot4( hash4( seed, hp[0], hp[1], hp[2], hp[3] ), d[0], d[1], d[2], d[3] ), f, value );
+            f = clampPositive( f ); f *= f; f *= f;
+            value = fmadd( gradDot4( gradHash4( seed, hp[0], hp[1], hp[2], hp[3] ), d[0], d[1], d[2], d[3] ), f, value );
         }
         {
-            float f = fmaxf_( f0, 0.0f ); f *= f; f *= f;
-            value = fmadd( gradDot4( hash4( seed, xP, yP, zP, wP ), d0[0], d0[1], d0[2], d0[3] ), f, value );
+            float f = clampPositive( f0 ); f *= f; f *= f;
+            value = fmadd( gradDot4( gradHash4( seed, xP, yP, zP, wP ), d0[0], d0[1], d0[2], d0[3] ), f, value );
         }
         return value;
     }
 
     // ---------------- SuperSimplex walks (Simplex.inl:291-936) ----------------
-    // vertex( hash, d[], falloff^4, first )
-    template<bool G = true, typename VTX>
+    // vertex( h, d[], falloff^4, first ): h is the vertex's gradHash, or with
+    // GRAD = false its hash
+    template<bool G = true, bool GRAD = true, typename VTX>
     FN2D void superWalk2( int32_t seed, float x, float y, VTX&& vertex )
     {
+        auto h2 = []( int32_t s, int32_t px, int32_t py ) { return GRAD ? gradHash2( s, px, py ) : hash2( s, px, py ); };
         constexpr double kSkew2 = 1.0 / ( kRoot3 + 1.0 );
         constexpr double kUnskew2 = -1.0 / ( kRoot3 + 3.0 );
         const float kFall = (float)( 2.0 / 3.0 );
@@ -266,14 +273,14 @@ namespace fn2d
         {
             float f = fb0; f *= f; f *= f;
             float d[2] = { dxB, dyB };
-            vertex( hash2( seed, xP, yP ), d, f, true );
+            vertex( h2( seed, xP, yP ), d, f, true );
         }
         {
             float f = fmadd( unskewDelta, (float)( -4.0 * ( kRoot3 + 2.0 ) / ( kRoot3 + 3.0 ) ), fb0 - kFall );
             f *= f; f *= f;
             const float o = (float)( 2 * kUnskew2 + 1 );
             float d[2] = { dxB - o, dyB - o };
-            vertex( hash2( seed, iadd( xP, kPX ), iadd( yP, kPY ) ), d, f, false );
+            vertex( h2( seed, iadd( xP, kPX ), iadd( yP, kPY ) ), d, f, false );
         }
         float xyDelta = fXY ? (float)( kUnskew2 + 1 ) : (float)-kUnskew2;
         dxB -= xyDelta;
@@ -288,7 +295,7 @@ namespace fn2d
             float f = fmaxf_( fnmadd( dx, dx, fnmadd( dy, dy, kFall ) ), 0.0f );
             f *= f; f *= f;
             float d[2] = { dx, dy };
-            vertex( hash2( seed, hx, hy ), d, f, false );
+            vertex( h2( seed, hx, hy ), d, f, false );
         }
         {
             int32_t hx = fXY ? iadd( xP, kPX ) : xP;
@@ -299,15 +306,16 @@ namespace fn2d
             float f = fmaxf_( fnmadd( dx, dx, fnmadd( dy, dy, kFall ) ), 0.0f );
             f *= f; f *= f;
             float d[2] = { dx, dy };
-            vertex( hash2( seed, hx, hy ), d, f, false );
+            vertex( h2( seed, hx, hy ), d, f, false );
         }
     }
 
     FN2D int32_t signBitIf( bool m ) { return m ? (int32_t)0x80000000u : 0; }
 
-    template<bool G = true, typename VTX>
+    template<bool G = true, bool GRAD = true, typename VTX>
     FN2D void superWalk3( int32_t seed, float x, float y, float z, VTX&& vertex )
     {
+        auto h3 = []( int32_t s, int32_t px, int32_t py, int32_t pz ) { return GRAD ? gradHash3( s, px, py, pz ) : hash3( s, px, py, pz ); };
         constexpr double kReflectUnskew3 = -1.0 / 2.0;
         constexpr double kTwiceUnskew3 = -1.0 / 4.0;
         const float kDistA = (float)( 3.0 / 4.0 );
@@ -325,9 +333,10 @@ namespace fn2d
             consider( xN, 0b001 ); consider( yN, 0b010 ); consider( zN, 0b100 );
             best += 0.125f - xyzN;
             consider( -zN, 0b011 ); consider( -yN, 0b101 ); consider( -xN, 0b110 );
-            if( bits & 1 ) { xB += 1.0f; dxS -= 1.0f; }
-            if( bits & 2 ) { yB += 1.0f; dyS -= 1.0f; }
-            if( bits & 4 ) { zB += 1.0f; dzS -= 1.0f; }
+            const float xUp = (float)( bits & 1 ), yUp = (float)( ( bits >> 1 ) & 1 ), zUp = (float)( ( bits >> 2 ) & 1 );
+            xB += xUp; dxS -= xUp;
+            yB += yUp; dyS -= yUp;
+            zB += zUp; dzS -= zUp;
         }
         int32_t xP = imul( floorToInt<G>( xB ), kPX ), yP = imul( floorToInt<G>( yB ), kPY ), zP = imul( floorToInt<G>( zB ), kPZ );
         float sum = dxS + dyS + dzS;
@@ -342,69 +351,71 @@ namespace fn2d
             stemA = fb - (float)( 3.0 / 4.0 * 0.5 );
             stemB = fb - (float)( 1.0 * 0.5 );
             float d[3] = { dxB, dyB, dzB };
-            vertex( hash3( seed, xP, yP, zP ), d, ( fb * fb ) * ( fb * fb ), true );
+            vertex( h3( seed, xP, yP, zP ), d, ( fb * fb ) * ( fb * fb ), true );
         }
-        auto pk = [&]( bool m, int32_t b, int32_t p ) { return iadd( b, m ? -p : p ); };
+        const int32_t xUp = iadd( xP, kPX ), yUp = iadd( yP, kPY ), zUp = iadd( zP, kPZ );
+        const int32_t xDn = isub( xP, kPX ), yDn = isub( yP, kPY ), zDn = isub( zP, kPZ );
+        // Each vertex steps along its axes, backwards where its difference (or
+        // coordinate: none of them can be -0) is negative. The falloffs are
+        // squared twice: max( -f, 0 ) does for min( f, 0 ).
         {   // <1,1,1>
-            bool sm = xyzN < 0.0f;
-            float off = fxor( (float)( 3 * kReflectUnskew3 + 1 ), signBitIf( sm ) );
-            float fb = fmaxf_( fmadd( off, coordSum, stemA ), 0.0f );
+            const int32_t s = signBit( xyzN ), m = negativeMask( xyzN );
+            float off = fxor( (float)( 3 * kReflectUnskew3 + 1 ), s );
+            float fb = clampPositive( fmadd( off, coordSum, stemA ) );
             float d[3] = { dxB - off, dyB - off, dzB - off };
-            vertex( hash3( seed, pk( sm, xP, kPX ), pk( sm, yP, kPY ), pk( sm, zP, kPZ ) ), d, ( fb * fb ) * ( fb * fb ), false );
+            vertex( h3( seed, bitSelect( m, xDn, xUp ), bitSelect( m, yDn, yUp ), bitSelect( m, zDn, zUp ) ), d, ( fb * fb ) * ( fb * fb ), false );
         }
         {   // <1,1,0>
-            bool sm = xyzN < zN;
-            int32_t s = signBitIf( sm );
+            const float t = xyzN - zN;
+            const int32_t s = signBit( t ), m = negativeMask( t );
             float off0 = fxor( (float)( 2 * kReflectUnskew3 ), s );
-            float fb = fminf_( fxor( dzB, s ) - stemB, 0.0f );
+            float fb = clampPositive( stemB - fxor( dzB, s ) );
             float d[3] = { dxB, dyB, dzB - off0 };
-            vertex( hash3( seed, pk( sm, xP, kPX ), pk( sm, yP, kPY ), zP ), d, ( fb * fb ) * ( fb * fb ), false );
+            vertex( h3( seed, bitSelect( m, xDn, xUp ), bitSelect( m, yDn, yUp ), zP ), d, ( fb * fb ) * ( fb * fb ), false );
         }
         {   // <1,0,1>
-            bool sm = xyzN < yN;
-            int32_t s = signBitIf( sm );
+            const float t = xyzN - yN;
+            const int32_t s = signBit( t ), m = negativeMask( t );
             float off0 = fxor( (float)( 2 * kReflectUnskew3 ), s );
-            float fb = fminf_( fxor( dyB, s ) - stemB, 0.0f );
+            float fb = clampPositive( stemB - fxor( dyB, s ) );
             float d[3] = { dxB, dyB - off0, dzB };
-            vertex( hash3( seed, pk( sm, xP, kPX ), yP, pk( sm, zP, kPZ ) ), d, ( fb * fb ) * ( fb * fb ), false );
+            vertex( h3( seed, bitSelect( m, xDn, xUp ), yP, bitSelect( m, zDn, zUp ) ), d, ( fb * fb ) * ( fb * fb ), false );
         }
         {   // <0,1,1>
-            bool sm = xyzN < xN;
-            int32_t s = signBitIf( sm );
+            const float t = xyzN - xN;
+            const int32_t s = signBit( t ), m = negativeMask( t );
             float off0 = fxor( (float)( 2 * kReflectUnskew3 ), s );
-            float fb = fminf_( fxor( dxB, s ) - stemB, 0.0f );
+            float fb = clampPositive( stemB - fxor( dxB, s ) );
             float d[3] = { dxB - off0, dyB, dzB };
-            vertex( hash3( seed, xP, pk( sm, yP, kPY ), pk( sm, zP, kPZ ) ), d, ( fb * fb ) * ( fb * fb ), false );
+            vertex( h3( seed, xP, bitSelect( m, yDn, yUp ), bitSelect( m, zDn, zUp ) ), d, ( fb * fb ) * ( fb * fb ), false );
         }
         {   // <1,0,0>
-            bool sm = xN < 0.0f;
-            int32_t s = signBitIf( sm );
+            const int32_t s = signBit( xN ), m = negativeMask( xN );
             float off0 = fxor( (float)kReflectUnskew3, s );
-            float fb = fmaxf_( fmadd( off0, coordSum, stemA ) + fxor( dxB, s ), 0.0f );
+            float fb = clampPositive( fmadd( off0, coordSum, stemA ) + fxor( dxB, s ) );
             float d[3] = { dxB + off0, dyB - off0, dzB - off0 };
-            vertex( hash3( seed, pk( sm, xP, kPX ), yP, zP ), d, ( fb * fb ) * ( fb * fb ), false );
+            vertex( h3( seed, bitSelect( m, xDn, xUp ), yP, zP ), d, ( fb * fb ) * ( fb * fb ), false );
         }
         {   // <0,1,0>
-            bool sm = yN < 0.0f;
-            int32_t s = signBitIf( sm );
+            const int32_t s = signBit( yN ), m = negativeMask( yN );
             float off0 = fxor( (float)kReflectUnskew3, s );
-            float fb = fmaxf_( fmadd( off0, coordSum, stemA ) + fxor( dyB, s ), 0.0f );
+            float fb = clampPositive( fmadd( off0, coordSum, stemA ) + fxor( dyB, s ) );
             float d[3] = { dxB - off0, dyB + off0, dzB - off0 };
-            vertex( hash3( seed, xP, pk( sm, yP, kPY ), zP ), d, ( fb * fb ) * ( fb * fb ), false );
+            vertex( h3( seed, xP, bitSelect( m, yDn, yUp ), zP ), d, ( fb * fb ) * ( fb * fb ), false );
         }
         {   // <0,0,1>
-            bool sm = zN < 0.0f;
-            int32_t s = signBitIf( sm );
+            const int32_t s = signBit( zN ), m = negativeMask( zN );
             float off0 = fxor( (float)kReflectUnskew3, s );
-            float fb = fmaxf_( fmadd( off0, coordSum, stemA ) + fxor( dzB, s ), 0.0f );
+            float fb = clampPositive( fmadd( off0, coordSum, stemA ) + fxor( dzB, s ) );
             float d[3] = { dxB - off0, dyB - off0, dzB + off0 };
-            vertex( hash3( seed, xP, yP, pk( sm, zP, kPZ ) ), d, ( fb * fb ) * ( fb * fb ), false );
+            vertex( h3( seed, xP, yP, bitSelect( m, zDn, zUp ) ), d, ( fb * fb ) * ( fb * fb ), false );
         }
     }
 
-    template<bool G = true, typename VTX>
+    template<bool G = true, bool GRAD = true, typename VTX>
     FN2D void superWalk4( int32_t seed, float x, float y, float z, float w, VTX&& vertex )
     {
+        auto h4 = []( int32_t s, int32_t px, int32_t py, int32_t pz, int32_t pw ) { return GRAD ? gradHash4( s, px, py, pz, pw ) : hash4( s, px, py, pz, pw ); };
         constexpr double kSkew4 = 1.0 / ( kRoot5 + 1.0 );
         constexpr double kUnskew4 = -1.0 / ( kRoot5 + 5.0 );
         constexpr double kTwiceUnskew4 = -1.0 / 5.0;
@@ -448,7 +459,7 @@ namespace fn2d
             float fb = fnmadd( dB[3], dB[3], fnmadd( dB[2], dB[2], fnmadd( dB[1], dB[1], fnmadd( dB[0], dB[0], kDistA ) ) ) ) * 0.5f;
             stemA = fb - (float)( 4.0 / 5.0 * 0.5 );
             stemB = fb - (float)( 6.0 / 5.0 * 0.5 );
-            vertex( hash4( seed, P[0], P[1], P[2], P[3] ), dB, ( fb * fb ) * ( fb * fb ), true );
+            vertex( h4( seed, P[0], P[1], P[2], P[3] ), dB, ( fb * fb ) * ( fb * fb ), true );
         }
         // One vertex: axes in `mask` move by +-1 with sign from `sm`.
         auto emit = [&]( bool sm, int mask, float offIn, float offOut, float fbPre ) {
@@ -464,7 +475,7 @@ namespace fn2d
                 hp[a] = in ? iadd( P[a], sm ? -prime[a] : prime[a] ) : P[a];
             }
             float fb = fmaxf_( fbPre, 0.0f );
-            vertex( hash4( seed, hp[0], hp[1], hp[2], hp[3] ), d, ( fb * fb ) * ( fb * fb ), false );
+            vertex( h4( seed, hp[0], hp[1], hp[2], hp[3] ), d, ( fb * fb ) * ( fb * fb ), false );
         };
         {   // <1,1,1,1>
             bool sm = xyzwN < 0.0f;

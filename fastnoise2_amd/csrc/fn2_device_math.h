@@ -137,6 +137,46 @@ namespace fn2d
     FN2D uint32_t umin( uint32_t a, uint32_t b ) { return a < b ? a : b; }
     FN2D uint32_t umax( uint32_t a, uint32_t b ) { return a > b ? a : b; }
 
+    // Selects as arithmetic on vector registers. A compare and a select on a
+    // scalar mask issue at half the rate of the rest (see gradDot3's tables),
+    // so where a < b decides several selects, the sign of a - b is spread over
+    // a mask once. a - b is negative exactly where a < b (denormals are kept);
+    // a NaN may go either way, and its results are NaN on both.
+    FN2D int32_t lessMask( float a, float b ) { return fbits( a - b ) >> 31; }
+    FN2D int32_t negativeMask( float a ) { return fbits( a ) >> 31; }
+    FN2D int32_t signBit( float a ) { return fbits( a ) & (int32_t)0x80000000u; }
+    // mask ? a : b per bit, as one v_bitop3_b32
+    FN2D int32_t bitSelect( int32_t mask, int32_t a, int32_t b )
+    {
+#if defined( __HIP_DEVICE_COMPILE__ )
+        return (int32_t)__builtin_amdgcn_bitop3_b32( (uint32_t)mask, (uint32_t)a, (uint32_t)b, 0xca );
+#else
+        return ( a & mask ) | ( b & ~mask );
+#endif
+    }
+    FN2D float bitSelect( int32_t mask, float a, float b ) { return ibits( bitSelect( mask, fbits( a ), fbits( b ) ) ); }
+    // 1.0f where the mask is set, else 0
+    FN2D float maskedOne( int32_t mask ) { return ibits( mask & 0x3f800000 ); }
+    // max( a, 0 ) of a value known to lie below 1 (or NaN, which gives 0):
+    // folds into the instruction that makes a as its clamp modifier
+    FN2D float clampPositive( float a )
+    {
+#if defined( __HIP_DEVICE_COMPILE__ )
+        return __builtin_amdgcn_fmed3f( a, 0.0f, 1.0f );
+#else
+        return a > 0.0f ? a : 0.0f;
+#endif
+    }
+    // the same value in a vector register: instructions with an operand in a
+    // scalar register issue at half rate
+    FN2D int32_t inVector( int32_t v )
+    {
+#if defined( __HIP_DEVICE_COMPILE__ )
+        asm( "" : "+v"( v ) );
+#endif
+        return v;
+    }
+
     // true when the predicate holds on every active lane of the wave (a host
     // build evaluates one point at a time: its own predicate)
 #if defined( __HIP_DEVICE_COMPILE__ )
@@ -175,6 +215,25 @@ namespace fn2d
     FN2D int32_t hash2( int32_t seed, int32_t x, int32_t y ) { return hashFinal( hashIn( seed, x, y ) ); }
     FN2D int32_t hash3( int32_t seed, int32_t x, int32_t y, int32_t z ) { return hashFinal( hashIn( seed, x, y, z ) ); }
     FN2D int32_t hash4( int32_t seed, int32_t x, int32_t y, int32_t z, int32_t w ) { return hashFinal( hashIn( seed, x, y, z, w ) ); }
+    // The product of a gradient's hash, times the size of a table entry: the
+    // bits of hashFinal that choose a gradient are bits 4 and up of
+    // m ^ ( m >> 15 ), an offset into the table with no shift left to do
+    static constexpr int kGradStride = 16;
+    FN2D int32_t gradHash2( int32_t seed, int32_t x, int32_t y ) { return imul( hashIn( seed, x, y ), imul( kHashMul, kGradStride ) ); }
+    FN2D int32_t gradHash3( int32_t seed, int32_t x, int32_t y, int32_t z ) { return imul( hashIn( seed, x, y, z ), imul( kHashMul, kGradStride ) ); }
+    FN2D int32_t gradHash4( int32_t seed, int32_t x, int32_t y, int32_t z, int32_t w ) { return imul( hashIn( seed, x, y, z, w ), imul( kHashMul, kGradStride ) ); }
+    // the table offset of a gradHash for `mask` = ( entries - 1 ) * kGradStride
+    FN2D int32_t gradOffset( int32_t m, int32_t mask )
+    {
+#if defined( __HIP_DEVICE_COMPILE__ )
+        // ( m ^ ( m >> 15 ) ) & mask as one v_bitop3_b32; the mask is no inline
+        // constant, and in a scalar register it would halve the issue rate
+        asm( "" : "+v"( mask ) );
+        return (int32_t)__builtin_amdgcn_bitop3_b32( (uint32_t)m, (uint32_t)isrl( m, 15 ), (uint32_t)mask, 0x28 );
+#else
+        return ( m ^ isrl( m, 15 ) ) & mask;
+#endif
+    }
     FN2D int32_t hashHB2( int32_t seed, int32_t x, int32_t y ) { return imul( hashIn( seed, x, y ), kHashMul ); }
     FN2D int32_t hashHB3( int32_t seed, int32_t x, int32_t y, int32_t z ) { return imul( hashIn( seed, x, y, z ), kHashMul ); }
     FN2D int32_t hashHB4( int32_t seed, int32_t x, int32_t y, int32_t z, int32_t w ) { return imul( hashIn( seed, x, y, z, w ), kHashMul ); }
@@ -233,11 +292,16 @@ namespace fn2d
     // -> 0.164, FBm(SuperSimplex) 3D 0.390 -> 0.302, FBm(Simplex) 2D 5 octaves
     // 0.152 -> 0.142 (against a scalar-unit path for waves in one cell that
     // this replaces), FBm(Perlin) 2D 0.156 -> 0.133, the serving tree 3D
-    // (with the warps' table, fn2_device_cellwarp.h) 0.968 -> 0.723.
+    // (with the warps' table, fn2_device_cellwarp.h) 0.968 -> 0.723. With the
+    // offsets straight from the hash product, and the lattices' and warps'
+    // selects as masks: 0.0565, 0.164, 0.164, 0.280, 0.137, 0.128, 0.701, and
+    // the same fractal as a 1024^2 tileable image (4D, whole call) 43.5 ->
+    // 39.8 us.
     // The 2-16 lanes that read one entry share it, and the entries of a 3D
     // table fill the 64 banks once, so reads do not conflict.
     // The kernels fill the tables they use before their first point
     // (fillTables).
+    // They take a gradHash: the entry's offset is a shift and a bitop3 away.
     struct alignas( 16 ) GradEntry2
     {
         int32_t signX, signY, swap, pad;
@@ -246,6 +310,12 @@ namespace fn2d
     {
         float x, y, z, w;
     };
+    static_assert( sizeof( GradEntry2 ) == kGradStride && sizeof( GradEntry ) == kGradStride, "table stride" );
+    template<class T>
+    __device__ __forceinline__ T gradEntry( const T* table, int32_t m, int entries )
+    {
+        return *reinterpret_cast<const T*>( reinterpret_cast<const char*>( table ) + gradOffset( m, ( entries - 1 ) * kGradStride ) );
+    }
     __device__ __forceinline__ GradEntry2* gradTable2()
     {
         __shared__ GradEntry2 t[8];
@@ -261,28 +331,23 @@ namespace fn2d
         __shared__ GradEntry t[32];
         return t;
     }
-    // mask ? a : b per bit, as one v_bitop3_b32
-    __device__ __forceinline__ float bitSelect( int32_t mask, float a, float b )
+    FN2D float gradDot2( int32_t m, float fx, float fy )
     {
-        return ibits( (int32_t)__builtin_amdgcn_bitop3_b32( (uint32_t)mask, (uint32_t)fbits( a ), (uint32_t)fbits( b ), 0xca ) );
-    }
-    FN2D float gradDot2( int32_t h, float fx, float fy )
-    {
-        const GradEntry2 e = gradTable2()[h & 7];
+        const GradEntry2 e = gradEntry( gradTable2(), m, 8 );
         fx = fxor( fx, e.signX );
         fy = fxor( fy, e.signY );
         return fmadd( 1.0f + kRoot2f, bitSelect( e.swap, fy, fx ), bitSelect( e.swap, fx, fy ) );
     }
     // the products are exact and all but two (three) of them zero, so the sum
     // rounds as the generic branch's does; only the sign of a zero may differ
-    FN2D float gradDot3( int32_t h, float fx, float fy, float fz )
+    FN2D float gradDot3( int32_t m, float fx, float fy, float fz )
     {
-        const GradEntry e = gradTable3()[h & 15];
+        const GradEntry e = gradEntry( gradTable3(), m, 16 );
         return fmadd( e.z, fz, fmadd( e.y, fy, e.x * fx ) );
     }
-    FN2D float gradDot4( int32_t h, float fx, float fy, float fz, float fw )
+    FN2D float gradDot4( int32_t m, float fx, float fy, float fz, float fw )
     {
-        const GradEntry e = gradTable4()[h & 31];
+        const GradEntry e = gradEntry( gradTable4(), m, 32 );
         return fmadd( e.w, fw, fmadd( e.z, fz, fmadd( e.y, fy, e.x * fx ) ) );
     }
     __device__ __forceinline__ void fillGradTable2( int e )
@@ -300,9 +365,9 @@ namespace fn2d
             gradTable4()[e] = { gradSelect4( e, 1, 0, 0, 0 ), gradSelect4( e, 0, 1, 0, 0 ), gradSelect4( e, 0, 0, 1, 0 ), gradSelect4( e, 0, 0, 0, 1 ) };
     }
 #else
-    FN2D float gradDot2( int32_t h, float fx, float fy ) { return gradSelect2( h, fx, fy ); }
-    FN2D float gradDot3( int32_t h, float fx, float fy, float fz ) { return gradSelect3( h, fx, fy, fz ); }
-    FN2D float gradDot4( int32_t h, float fx, float fy, float fz, float fw ) { return gradSelect4( h, fx, fy, fz, fw ); }
+    FN2D float gradDot2( int32_t m, float fx, float fy ) { return gradSelect2( gradOffset( m, 7 * kGradStride ) / kGradStride, fx, fy ); }
+    FN2D float gradDot3( int32_t m, float fx, float fy, float fz ) { return gradSelect3( gradOffset( m, 15 * kGradStride ) / kGradStride, fx, fy, fz ); }
+    FN2D float gradDot4( int32_t m, float fx, float fy, float fz, float fw ) { return gradSelect4( gradOffset( m, 31 * kGradStride ) / kGradStride, fx, fy, fz, fw ); }
 #endif
 
     // ScaleOutput (BasicGenerators.inl:27-30): scale = (1/(max-min)) * rangeScale folded on the host

@@ -78,6 +78,7 @@ namespace fn2i
     template<int D, int LEAF = -1, bool G = true>
     FN2D float leafRaw( int op, int32_t seed, const float* x )
     {
+        seed = inVector( seed );   // xored into every corner's hash
         if constexpr( opIn<LEAF, fn2::OP_PERLIN>() )
             if( LEAF >= 0 || op == fn2::OP_PERLIN )
             {
