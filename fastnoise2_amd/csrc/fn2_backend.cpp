@@ -137,7 +137,7 @@ namespace fn2
         {
             GenArgs copy = a;
             void* params[] = { &copy };
-            const unsigned grid = fn2_grid_for( a.total, k->blocksPerCU );
+            const unsigned grid = k->wide && a.kind == SRC_GRID ? fn2_wide_grid_for( a.total, a.minmax != nullptr ) : fn2_grid_for( a.total, k->blocksPerCU );
             if( blocks ) *blocks = grid;
             if( direct && grid <= (unsigned)kRangeDirectBlocks ) copy.minmax = direct;
             return hipModuleLaunchKernel( k->single, grid, 1, 1, 256, 1, 1, 0, stream, params, nullptr );

@@ -113,6 +113,24 @@ namespace fn2
             return false;
         }
 
+        // A program cheap enough that writing its values is what takes the time:
+        // at most 8 instructions without a noise, warp, division, power or root (the
+        // checkerboard's 12 operations per point take 4 points per lane, an
+        // 8-instruction sum of them stays below the writes too)
+        bool Wide( const DeviceProgram& p )
+        {
+            if( p.ins.size() > 8 ) return false;
+            for( const Ins& in : p.ins )
+                switch( in.op )
+                {
+                case OP_CONST: case OP_MOV: case OP_MOV_VEC: case OP_ADD: case OP_SUB: case OP_MUL: case OP_MIN: case OP_MAX: case OP_ABS:
+                case OP_SCALE: case OP_SCALE_AXES: case OP_ADD_VEC: case OP_SUB_VEC: case OP_MUL_VEC: case OP_GRADIENT_AXIS:
+                case OP_CHECKERBOARD: case OP_WHITE: break;
+                default: return false;
+                }
+            return true;
+        }
+
         // The LDS tables (kTable*) the program's instructions read
         int Tables( const DeviceProgram& p )
         {
@@ -149,6 +167,7 @@ namespace fn2
                  "static constexpr bool kFresh = true;\n"
                  "static constexpr int kDims = " << p.dims << ";\n"
                  "static constexpr bool kBricks = " << ( PrunedCellular( p ) ? "true" : "false" ) << ";\n"
+                 "static constexpr bool kWide = " << ( Wide( p ) ? "true" : "false" ) << ";\n"
                  "static constexpr int kTables = " << Tables( p ) << ";\n"
                  "__device__ __forceinline__ float operator()( const fn2::GenArgs& a, float* R ) const {\n";
             // long programs get a register fence between instructions: measured
@@ -241,6 +260,7 @@ namespace fn2
                 return false;
             }
             k.module = mod;
+            k.wide = Wide( p );
             if( hipModuleOccupancyMaxActiveBlocksPerMultiprocessor( &k.blocksPerCU, k.single, 256, 0 ) != hipSuccess )
             {
                 (void)hipGetLastError();

@@ -15,6 +15,7 @@ namespace fn2
         hipFunction_t queue = nullptr;    // fn2_jit_queue( jobs, tileJob, tileBase, nTiles, counter )
         int blocksPerCU = 0;              // resident 256-thread blocks of `single` per CU
         int queueBlocksPerCU = 0;         // the same for `queue`
+        bool wide = false;                // a cheap program: grid requests write four points per lane
         int singleRegs = 0;               // VGPRs per lane of `single`, as the runtime reports them
         int singleScratch = 0;            // private (scratch) bytes per lane of `single`
     };

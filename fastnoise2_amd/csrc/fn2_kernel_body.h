@@ -18,7 +18,20 @@ namespace fn2k
     // Output stores of whole wave rows (64 consecutive floats): each value
     // is written once and never read back by the kernel, so they go out as
     // streaming (non-temporal) stores
-    __device__ __forceinline__ void storeOut( float* p, float v ) { __builtin_nontemporal_store( v, p ); }
+    // (an output address read from a job record is a generic pointer: said to
+    // be global, the store is no flat one)
+    __device__ __forceinline__ void storeOut( float* p, float v )
+    {
+        __builtin_nontemporal_store( v, (__attribute__( ( address_space( 1 ) ) ) float*)p );
+    }
+
+    // Adds a value to a lane's range; a NaN adds nothing (fminf and fmaxf
+    // return the other operand)
+    __device__ __forceinline__ void widen( float v, float& mn, float& mx )
+    {
+        mn = fminf( mn, v );
+        mx = fmaxf( mx, v );
+    }
 
     // BLOCK: the most threads a block of the kernel has (its launch bound);
     // the block may have fewer, any multiple of 64.
@@ -157,12 +170,65 @@ namespace fn2k
                 // streaming stores went out piece by piece (2.8 times the
                 // output's bytes on the warped cellular 256^3 grid)
                 a.out[( z * ny + y ) * nx + x] = v;
-                if( v == v )
-                {
-                    mn = fminf( mn, v );
-                    mx = fmaxf( mx, v );
-                }
+                widen( v, mn, mx );
             }
+        }
+    }
+
+    // A grid request of a cheap program (Prog::kWide), four consecutive points
+    // per lane: one 16-byte store for them, and the division of the index
+    // and the coordinates but x shared unless the row ends among them. Bounded
+    // by the writes: with a point per lane these kernels spent about 100
+    // cycles of a SIMD per wave and point, most of it on the index, which was
+    // as long as the writes took. One point per lane -> four on MI355X, GB/s
+    // in turn into several buffers: checkerboard 4096^2 3921 -> 5366, 8192^2
+    // 4385 -> 6600, 16384^2 5327 -> 6944; white noise 8192^2 3790 -> 6376; a
+    // constant 8192^2 4890 -> 6180 (a fill of 256 MB: 6700). The output has to
+    // lie on 16 bytes; programs with more to do per point gain nothing and
+    // would need four points' registers.
+    // RANGED: the call wants its range (a copy without it saves a fifth of
+    // the instructions).
+    template<int BLOCK, bool RANGED, class Prog>
+    __device__ __forceinline__ void generateWide( const fn2::GenArgs& a, Prog prog, float& mn, float& mx )
+    {
+        typedef float Vec4 __attribute__( ( ext_vector_type( 4 ) ) );
+        constexpr int D = Prog::kDims;
+        const uint32_t total = (uint32_t)a.total, groups = total / 4;
+        // a contiguous run of whole rounds per block
+        const uint32_t run = ( groups + gridDim.x * BLOCK - 1 ) / ( gridDim.x * BLOCK ) * BLOCK;
+        const uint32_t begin = blockIdx.x * run, end = begin + run < groups ? begin + run : groups;
+        for( uint32_t g = begin + threadIdx.x; g < end; g += BLOCK )
+        {
+            RegFile first;
+            startPositionD<D, false>( a, 4 * g, first.R );
+            const uint32_t x = 4 * g - fastDiv( a.div[0], 4 * g ) * a.div[0].d;
+            const bool row = x + 3 < a.div[0].d;
+            Vec4 v;
+#pragma unroll
+            for( int k = 0; k < 4; k++ )
+            {
+                RegFile fresh;
+                if( row )
+                {
+                    fresh.R[0] = fmadd( (float)(int32_t)( x + k ), a.step[0], a.offset[0] );
+#pragma unroll
+                    for( int ax = 1; ax < D; ax++ ) fresh.R[ax] = first.R[ax];
+                }
+                else startPositionD<D, false>( a, 4 * g + k, fresh.R );
+                v[k] = prog( a, fresh.R );
+                if constexpr( RANGED ) widen( v[k], mn, mx );
+            }
+            // a plain store: streaming ones were slower (WideGridFor's figures)
+            *reinterpret_cast<Vec4*>( a.out + 4 * g ) = v;
+        }
+        const uint32_t rest = 4 * groups + threadIdx.x;
+        if( blockIdx.x == 0 && rest < total )
+        {
+            RegFile fresh;
+            startPositionD<D, false>( a, rest, fresh.R );
+            const float v = prog( a, fresh.R );
+            storeOut( a.out + rest, v );
+            widen( v, mn, mx );
         }
     }
 
@@ -174,26 +240,31 @@ namespace fn2k
         float mn = __builtin_inff(), mx = -__builtin_inff();
         auto emit = [&]( uint32_t i, float v ) {
             storeOut( a.out + i, v );
-            if( v == v )
-            {
-                mn = fminf( mn, v );
-                mx = fmaxf( mx, v );
-            }
+            widen( v, mn, mx );
         };
         const uint32_t total = (uint32_t)a.total;
         const uint32_t stride = gridDim.x * BLOCK;
         if constexpr( Prog::kFresh )
         {
-            bool bricks = false;
+            bool done = false;
             if constexpr( Prog::kBricks && ( Prog::kDims == 2 || Prog::kDims == 3 ) )
             {
                 if( a.kind == fn2::SRC_GRID && a.dims == Prog::kDims )
                 {
                     generateBricks<BLOCK, Prog::kDims>( a, prog, mn, mx );
-                    bricks = true;
+                    done = true;
                 }
             }
-            if( !bricks )
+            if constexpr( Prog::kWide )
+            {
+                if( a.kind == fn2::SRC_GRID && a.dims == Prog::kDims && ( reinterpret_cast<uint64_t>( a.out ) & 15 ) == 0 )
+                {
+                    if( a.minmax ) generateWide<BLOCK, true>( a, prog, mn, mx );
+                    else generateWide<BLOCK, false>( a, prog, mn, mx );
+                    done = true;
+                }
+            }
+            if( !done )
             {
                 for( uint32_t i = blockIdx.x * BLOCK + threadIdx.x; i < total; i += stride )
                 {
@@ -227,11 +298,7 @@ namespace fn2k
         float mn = __builtin_inff(), mx = -__builtin_inff();
         auto emit = [&]( uint32_t i, float v ) {
             storeOut( a.out + i, v );
-            if( v == v )
-            {
-                mn = fminf( mn, v );
-                mx = fmaxf( mx, v );
-            }
+            widen( v, mn, mx );
         };
         const uint32_t total = (uint32_t)a.total;
         const uint32_t base = first + threadIdx.x;
@@ -345,11 +412,7 @@ namespace fn2k
             const int ppt = a.ppt;
             auto emit = [&]( uint32_t i, float v ) {
                 storeOut( a.out + i, v );
-                if( v == v )
-                {
-                    mn = fminf( mn, v );
-                    mx = fmaxf( mx, v );
-                }
+                widen( v, mn, mx );
             };
             if constexpr( Prog::kFresh )
             {

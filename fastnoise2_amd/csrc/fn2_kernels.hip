@@ -213,6 +213,24 @@ namespace
         return (unsigned)( need < cap ? need : cap );
     }
 
+    // Blocks of a single-call kernel of a cheap program, which writes four
+    // points per lane and round (4 KiB a block) and takes a contiguous run of
+    // rounds per block (fn2k::generateWide): 4096 blocks or runs of four
+    // rounds, and of two beyond 64 MB, where short runs keep the blocks at
+    // work at one time writing close together. Measured on MI355X, GB/s of
+    // checkerboards of 64 MB / 256 MB / 1 GB in turn into several buffers: one
+    // point per lane 3921 / 4385 / 5327; 4096 blocks 5356 / 5696 / 5570, 16384
+    // 4696 / 6031 / 5378, 32768 4680 / 6532 / 5468, 65536 4670 / 5700 / 5883 (a
+    // fill of 256 MB: 6715). With a range every block costs a pair to reduce:
+    // at most 8192.
+    unsigned WideGridFor( int64_t total, bool ranged )
+    {
+        const int64_t rounds = std::max<int64_t>( 1, ( total / 4 + kBlock - 1 ) / kBlock );
+        const int64_t run = rounds <= 16384 ? 4 : 2;
+        const int64_t blocks = std::max( std::min<int64_t>( rounds, 4096 ), ( rounds + run - 1 ) / run );
+        return (unsigned)( ranged ? std::min<int64_t>( blocks, 8192 ) : blocks );
+    }
+
     // Resident blocks per CU of an interpreter variant at a register-file size
     template<class K>
     int ResidentBlocks( K kernel, size_t lds )
@@ -256,6 +274,11 @@ extern "C" {
 unsigned fn2_grid_for( int64_t total, int blocksPerCU )
 {
     return GridFor( total, blocksPerCU );
+}
+
+unsigned fn2_wide_grid_for( int64_t total, int ranged )
+{
+    return WideGridFor( total, ranged != 0 );
 }
 
 // threads per block of the batched kernel: a job with ppt points per lane

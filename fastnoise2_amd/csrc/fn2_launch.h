@@ -34,6 +34,9 @@ int fn2_launch_generate( const fn2::GenArgs* args, int dimMask, int featMask, hi
 // blocks of a single-call launch over `total` points (also used for the
 // run-time specialised kernels), at most kMaxCallBlocks
 unsigned fn2_grid_for( int64_t total, int blocksPerCU );
+// the same for grid requests of cheap programs (JitKernel::wide); at most
+// kMaxCallBlocks when the call has a range record
+unsigned fn2_wide_grid_for( int64_t total, int ranged );
 // interpreter launch over a batch of jobs (block b runs job dBlockJob[b])
 int fn2_launch_generate_batch( const fn2::GenArgs* dJobs, const int32_t* dBlockJob, const uint32_t* dBlockBase, int nBlocks, int dimMask, int featMask,
                                int regs, hipStream_t stream );
