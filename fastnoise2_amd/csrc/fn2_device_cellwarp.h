@@ -15,6 +15,18 @@ namespace fn2d
         else if constexpr( D == 3 ) return hashHB3( seed, c[0], c[1], c[2] );
         else return hashHB4( seed, c[0], c[1], c[2], c[3] );
     }
+    // bits 1-10 of b as a number minus 511.5: set into the mantissa of 2^22
+    // (whose last bit counts halves), which is subtracted again. Exact, and
+    // three full-rate instructions instead of a half-rate conversion and more.
+    FN2D float centredField( int32_t b )
+    {
+#if defined( __HIP_DEVICE_COMPILE__ )
+        const int32_t mask = inVector( 0x7fe ), one = inVector( 0x4a800000 );
+        return ibits( (int32_t)__builtin_amdgcn_bitop3_b32( (uint32_t)b, (uint32_t)mask, (uint32_t)one, 0xea ) ) - ( 4194304.0f + 511.5f );
+#else
+        return ibits( ( b & 0x7fe ) | 0x4a800000 ) - ( 4194304.0f + 511.5f );
+#endif
+    }
     // jittered cell-point direction from the hash (Cellular.inl:55-56, 141-143, 239-242)
     template<int D> FN2D void cellVector( int32_t h, float* v )
     {
@@ -25,9 +37,10 @@ namespace fn2d
         }
         else if constexpr( D == 3 )
         {
-            v[0] = (float)( h & 0x3ff ) - 0x3ff / 2.0f;
-            v[1] = (float)( ( h >> 11 ) & 0x3ff ) - 0x3ff / 2.0f;
-            v[2] = (float)isrl( h, 22 ) - 0x3ff / 2.0f;
+            h = inVector( h );   // else h + h becomes a second multiplication
+            v[0] = centredField( iadd( h, h ) );
+            v[1] = centredField( isrl( h, 10 ) );
+            v[2] = centredField( isrl( h, 21 ) );
         }
         else
         {
@@ -287,9 +300,9 @@ namespace fn2d
             // min / max steps above (a NaN distance never displaces a slot, and
             // no slot becomes NaN), without canonicalising their operands.
             const uint32_t nb = (uint32_t)fbits( nd );
-            if constexpr( SLOTS > 3 ) key[3] = umax( umin( key[3], nb ), key[2] );
-            if constexpr( SLOTS > 2 ) key[2] = umax( umin( key[2], nb ), key[1] );
-            if constexpr( SLOTS > 1 ) key[1] = umax( umin( key[1], nb ), key[0] );
+            if constexpr( SLOTS > 3 ) key[3] = umed3( key[2], key[3], nb );
+            if constexpr( SLOTS > 2 ) key[2] = umed3( key[1], key[2], nb );
+            if constexpr( SLOTS > 1 ) key[1] = umed3( key[0], key[1], nb );
             key[0] = umin( key[0], nb );
         }
 #pragma unroll
@@ -321,47 +334,49 @@ namespace fn2d
         return waves[threadIdx.x >> 6];
     }
 
-    // The table walks' common part. c[a]: the lane's first walk cell on
-    // axis a (the rounded position - 1); first[a]: the first active lane's.
-    // When every active lane has c within one of first on every axis and
-    // the same seed, fills the wave's table for the box of cells first - 1
-    // .. first + 3 (table coordinate t = cell - first + 1) and returns true;
-    // else returns false, having written nothing. HASH: also keep each
-    // cell's hash (CellularValue returns it).
+    // The table walks' common part. c[a]: the lane's first walk cell on axis a
+    // (the rounded position - 1). When the active lanes' c lie within one of
+    // the first active lane's on every axis and the seed is the same, fills
+    // the wave's table and returns true: the cell `origin + t` has its entry
+    // at t[0] + 5 t[1] + 25 t[2], for a box of 5 cells a side around the first
+    // lane's walk, or, in 3D where the c take at most two values per axis (most
+    // grid bricks), one of 4 cells a side, which the 64 lanes fill in one
+    // round instead of two. Else returns false, having written nothing. HASH:
+    // also keep each cell's hash (CellularValue returns it).
     template<int D, bool HASH>
-    __device__ __forceinline__ bool fillCellTable( const CellParams& cp, const float* pos, int32_t* c, int32_t* first )
+    __device__ __forceinline__ bool fillCellTable( const CellParams& cp, const float* pos, int32_t* c, int32_t* origin )
     {
-        constexpr int kEntries = D == 2 ? 25 : 125;
         const int32_t prime[3] = { kPX, kPY, kPZ };
         bool near = cp.seed == __builtin_amdgcn_readfirstlane( cp.seed );
+        bool tight = D == 3 && near;
+        int32_t first[D], below[D];
 #pragma unroll
         for( int a = 0; a < D; a++ )
         {
             c[a] = iadd( roundToInt( pos[a] ), -1 );
             first[a] = __builtin_amdgcn_readfirstlane( c[a] );
-            // c - first in {-1, 0, 1}, in wrapping arithmetic
-            near = near && (uint32_t)c[a] - (uint32_t)first[a] + 1u <= 2u;
+            // differences in wrapping arithmetic
+            const int32_t diff = isub( c[a], first[a] );
+            near = near && (uint32_t)iadd( diff, 1 ) <= 2u;
+            if constexpr( D == 3 )
+            {
+                below[a] = __any( diff < 0 ) ? 1 : 0;
+                tight = tight && (uint32_t)iadd( diff, below[a] ) <= 1u;
+            }
         }
-        if( !waveAll( near ) ) return false;
+        if constexpr( D == 3 ) tight = waveAll( tight );
+        if( !tight && !waveAll( near ) ) return false;
 
         CellEntry* tbl = cellTable<D>();
         const uint64_t active = __ballot( 1 );
         const uint32_t rank = __builtin_amdgcn_mbcnt_hi( (uint32_t)( active >> 32 ), __builtin_amdgcn_mbcnt_lo( (uint32_t)active, 0u ) );
         const uint32_t lanes = (uint32_t)__builtin_popcountll( active );
-        // the previous use of the table by this wave is over
-        __builtin_amdgcn_fence( __ATOMIC_ACQ_REL, "wavefront" );
-        __builtin_amdgcn_wave_barrier();
-        for( uint32_t e = rank; e < (uint32_t)kEntries; e += lanes )
-        {
+        auto fill = [&]( const int32_t* t ) {
             int32_t hc[D];
-            uint32_t rest = e;
+            int32_t at = t[0] + 5 * t[1];
+            if constexpr( D == 3 ) at += 25 * t[D - 1];
 #pragma unroll
-            for( int a = 0; a < D; a++ )
-            {
-                const int32_t t = (int32_t)( rest % 5u );
-                rest /= 5u;
-                hc[a] = imul( iadd( first[a], t - 1 ), prime[a] );
-            }
+            for( int a = 0; a < D; a++ ) hc[a] = imul( iadd( origin[a], t[a] ), prime[a] );
             const int32_t h = cellHash<D>( cp.seed, hc );
             float v[D];
             cellVector<D>( h, v );
@@ -370,8 +385,31 @@ namespace fn2d
             entry.v[1] = v[1];
             entry.v[2] = D > 2 ? v[D - 1] : 0.0f;
             entry.invMag = invSqrtCell<D>( cellMagSq<D>( v ) );
-            tbl[e] = entry;
-            if constexpr( HASH ) cellHashTable<D>()[e] = h;
+            tbl[at] = entry;
+            if constexpr( HASH ) cellHashTable<D>()[at] = h;
+        };
+        // the previous use of the table by this wave is over
+        __builtin_amdgcn_fence( __ATOMIC_ACQ_REL, "wavefront" );
+        __builtin_amdgcn_wave_barrier();
+        if( tight )
+        {
+#pragma unroll
+            for( int a = 0; a < D; a++ ) origin[a] = isub( first[a], below[a] );
+            for( uint32_t e = rank; e < 64u; e += lanes )
+            {
+                const int32_t t[3] = { (int32_t)( e & 3u ), (int32_t)( ( e >> 2 ) & 3u ), (int32_t)( e >> 4 ) };
+                fill( t );
+            }
+        }
+        else
+        {
+#pragma unroll
+            for( int a = 0; a < D; a++ ) origin[a] = isub( first[a], 1 );
+            for( uint32_t e = rank; e < ( D == 2 ? 25u : 125u ); e += lanes )
+            {
+                const int32_t t[3] = { (int32_t)( e % 5u ), (int32_t)( ( e / 5u ) % 5u ), (int32_t)( e / 25u ) };
+                fill( t );
+            }
         }
         __builtin_amdgcn_fence( __ATOMIC_ACQ_REL, "wavefront" );
         __builtin_amdgcn_wave_barrier();
@@ -397,8 +435,8 @@ namespace fn2d
     {
         using Order = MirroredCellOrder<D>;
         constexpr Order order;
-        int32_t c[D], first[D];
-        if( !fillCellTable<D, false>( cp, pos, c, first ) ) return false;
+        int32_t c[D], origin[D];
+        if( !fillCellTable<D, false>( cp, pos, c, origin ) ) return false;
         const CellEntry* tbl = cellTable<D>();
 
         // the lane's mirrored columns: table offsets and cell positions
@@ -408,7 +446,7 @@ namespace fn2d
         for( int a = 0; a < D; a++ )
         {
             const int32_t scale = a == 0 ? 1 : a == 1 ? 5 : 25;
-            const int32_t t0 = (int32_t)( (uint32_t)c[a] - (uint32_t)first[a] + 1u );   // 0..2
+            const int32_t t0 = isub( c[a], origin[a] );   // 0..2
             T[a][0] = t0 * scale;
             T[a][1] = T[a][0] + scale;
             T[a][2] = T[a][1] + scale;
@@ -458,9 +496,9 @@ namespace fn2d
             for( int a = 0; a < D; a++ ) d[a] = fmadd( cell.v[a], invMag, rel[a][o[a]] );
             const float nd = calcDistance<D>( cp.distFunc, false, d, cp.minkowskiP );
             const uint32_t nb = (uint32_t)fbits( nd );
-            if constexpr( SLOTS > 3 ) key[3] = umax( umin( key[3], nb ), key[2] );
-            if constexpr( SLOTS > 2 ) key[2] = umax( umin( key[2], nb ), key[1] );
-            if constexpr( SLOTS > 1 ) key[1] = umax( umin( key[1], nb ), key[0] );
+            if constexpr( SLOTS > 3 ) key[3] = umed3( key[2], key[3], nb );
+            if constexpr( SLOTS > 2 ) key[2] = umed3( key[1], key[2], nb );
+            if constexpr( SLOTS > 1 ) key[1] = umed3( key[0], key[1], nb );
             key[0] = umin( key[0], nb );
         }
 #pragma unroll
@@ -477,8 +515,8 @@ namespace fn2d
     template<int D, int SLOTS>
     __device__ __forceinline__ bool cellularDistancesTableAll( const CellParams& cp, const float* pos, float* dist )
     {
-        int32_t c[D], first[D];
-        if( !fillCellTable<D, true>( cp, pos, c, first ) ) return false;
+        int32_t c[D], origin[D];
+        if( !fillCellTable<D, true>( cp, pos, c, origin ) ) return false;
         const CellEntry* tbl = cellTable<D>();
         const int32_t* htbl = cellHashTable<D>();
         int32_t T[D];
@@ -487,7 +525,7 @@ namespace fn2d
         for( int a = 0; a < D; a++ )
         {
             const int32_t scale = a == 0 ? 1 : a == 1 ? 5 : 25;
-            T[a] = (int32_t)( (uint32_t)c[a] - (uint32_t)first[a] + 1u ) * scale;   // the lane's first cell
+            T[a] = isub( c[a], origin[a] ) * scale;   // the lane's first cell
             float fc = (float)c[a];
             rel[a][0] = fc - pos[a];
             fc = fc + 1.0f;
@@ -529,8 +567,8 @@ namespace fn2d
     template<int D>
     __device__ __forceinline__ bool cellularLookupTable( const CellParams& cp, const float* pos, float* cellPos )
     {
-        int32_t c[D], first[D];
-        if( !fillCellTable<D, true>( cp, pos, c, first ) ) return false;
+        int32_t c[D], origin[D];
+        if( !fillCellTable<D, true>( cp, pos, c, origin ) ) return false;
         const CellEntry* tbl = cellTable<D>();
         const int32_t* htbl = cellHashTable<D>();
         int32_t T[D];
@@ -539,7 +577,7 @@ namespace fn2d
         for( int a = 0; a < D; a++ )
         {
             const int32_t scale = a == 0 ? 1 : a == 1 ? 5 : 25;
-            T[a] = (int32_t)( (uint32_t)c[a] - (uint32_t)first[a] + 1u ) * scale;   // the lane's first cell
+            T[a] = isub( c[a], origin[a] ) * scale;   // the lane's first cell
             F[a][0] = (float)c[a];
             F[a][1] = F[a][0] + 1.0f;
             F[a][2] = F[a][1] + 1.0f;
@@ -581,8 +619,8 @@ namespace fn2d
     template<int D>
     __device__ __forceinline__ bool cellularValueTable( const CellParams& cp, const float* pos, int valueIndex, float& result )
     {
-        int32_t c[D], first[D];
-        if( !fillCellTable<D, true>( cp, pos, c, first ) ) return false;
+        int32_t c[D], origin[D];
+        if( !fillCellTable<D, true>( cp, pos, c, origin ) ) return false;
         const CellEntry* tbl = cellTable<D>();
         const int32_t* htbl = cellHashTable<D>();
         int32_t T[D];
@@ -591,7 +629,7 @@ namespace fn2d
         for( int a = 0; a < D; a++ )
         {
             const int32_t scale = a == 0 ? 1 : a == 1 ? 5 : 25;
-            T[a] = (int32_t)( (uint32_t)c[a] - (uint32_t)first[a] + 1u ) * scale;   // the lane's first cell
+            T[a] = isub( c[a], origin[a] ) * scale;   // the lane's first cell
             F[a][0] = (float)c[a] - pos[a];
             F[a][1] = F[a][0] + 1.0f;
             F[a][2] = F[a][1] + 1.0f;
@@ -733,7 +771,7 @@ namespace fn2d
         auto hxR = [&]( int a, int col ) { return hx[a][col]; };
         uint32_t key[2] = { 0x7f800000u, 0x7f800000u };   // +inf
         auto insert = [&]( uint32_t nb ) {
-            if constexpr( SLOTS > 1 ) key[1] = umax( umin( key[1], nb ), key[0] );
+            if constexpr( SLOTS > 1 ) key[1] = umed3( key[0], key[1], nb );
             key[0] = umin( key[0], nb );
         };
         // the near octant, for every lane
@@ -919,9 +957,20 @@ namespace fn2d
         for( int i = 1; i < 4; i++ ) { a = i0 == i ? dist[i] : a; b = i1 == i ? dist[i] : b; }
         if( distFunc == 0 )
         {
-            a *= invSqrt( a );
-            // the same slot twice takes the root twice, as the reference does
-            b = i0 == i1 ? a * invSqrt( a ) : b * invSqrt( b );
+            // the general routines' scaling and division take about 80 cycles
+            // of a SIMD per root more than invSqrtPos, which every distance
+            // in [2^-60, 2^61) may take (test_gpu_cell_math.py)
+            if( waveAll( invSqrtPosHolds( a ) && invSqrtPosHolds( b ) ) )
+            {
+                a *= invSqrtPos( a );
+                // the same slot twice takes the root twice, as the reference does
+                b = i0 == i1 ? a * invSqrtPos( a ) : b * invSqrtPos( b );
+            }
+            else
+            {
+                a *= invSqrt( a );
+                b = i0 == i1 ? a * invSqrt( a ) : b * invSqrt( b );
+            }
             if( i0 == i1 ) a = b;
         }
         (void)maxDist;

@@ -68,7 +68,7 @@ __global__ void fn2_selftest_math( int op, const float* in, float* out, int n )
     {
         float x = in[i];
         out[i] = op == 0 ? sqrtPosRN( x ) : op == 1 ? recipPosRN( x ) : op == 2 ? invSqrtPos( x ) : op == 3 ? invSqrt( x )
-               : op == 4 ? __builtin_amdgcn_sqrtf( x ) : sqrtPosRNFromBelow( x );
+               : op == 4 ? __builtin_amdgcn_sqrtf( x ) : op == 5 ? sqrtPosRNFromBelow( x ) : invSqrtCell<3>( x );
     }
 }
 
