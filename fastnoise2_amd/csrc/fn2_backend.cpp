@@ -662,7 +662,23 @@ namespace fn2
         a.resultReg = dp->resultReg;
 
         const bool devOut = IsDevicePointer( out );
+        // A host output too short for the staging ring is written by the kernel
+        // into pinned memory: its stores cross PCIe while it computes, where
+        // device memory and a copy add the copy's submission and its transfer
+        // after the kernel. 2D Simplex fractal of 5 octaves with its range,
+        // copied / in place, us: 1 K floats 29.7 / 19.3, 64 K 41 / 30, 256 K
+        // 82 / 74; above, the ring's copies by several threads are as fast (1 M
+        // 189 / 242 with one thread's copy, 2049 x 1023 335 / 345 with several).
+        // The kernels that write bricks keep the copy: their stores would cross
+        // PCIe 16 bytes at a time.
+        const bool pinnedOut = !devOut && total < kStagedMinFloats && !( spec.kind == FN2_SOURCE_GRID && JitWalksBricks( *dp ) );
         if( devOut ) a.out = out;
+        else if( pinnedOut )
+        {
+            if( !c->hOut && !HipOk( hipHostMalloc( (void**)&c->hOut, (size_t)kStagedMinFloats * sizeof( float ), hipHostMallocDefault ), "hipHostMalloc(output)" ) )
+                return fail( tLastError );
+            a.out = c->hOut;
+        }
         else
         {
             if( !c->Reserve( c->dOut, c->outCap, (size_t)total ) ) return fail( tLastError );
@@ -697,7 +713,7 @@ namespace fn2
         }
 
         if( !c->LaunchRanged( a, dp, c->stream ) ) return fail( tLastError );
-        if( !devOut )
+        if( !devOut && !pinnedOut )
         {
             if( total >= kStagedMinFloats )
             {
@@ -709,6 +725,7 @@ namespace fn2
             }
         }
         if( !HipOk( hipStreamSynchronize( c->stream ), "generator kernel" ) ) return fail( tLastError );
+        if( pinnedOut ) memcpy( out, c->hOut, (size_t)total * sizeof( float ) );
 
         c->Range( r.min, r.max );
         return r;

@@ -49,6 +49,7 @@ namespace fn2
         int32_t* dKeys = nullptr;   // a call's range record: kMaxCallBlocks pairs
         int32_t* hKeys = nullptr;   // pinned: kRangeDirectBlocks pairs, written by the kernels
         hipEvent_t ev0 = nullptr, ev1 = nullptr;
+        float* hOut = nullptr;      // pinned, kStagedMinFloats
         float* hStage = nullptr;    // pinned ring: kStageSlots chunks of kStageChunkFloats
         hipEvent_t evStage[kStageSlots] = {};
 

@@ -467,6 +467,8 @@ namespace fn2
         return Manager().State( p, variant, nullptr );
     }
 
+    bool JitWalksBricks( const DeviceProgram& p ) { return PrunedCellular( p ); }
+
     bool JitHasFusedFractal( const DeviceProgram& p )
     {
         for( const Ins& in : p.ins )

@@ -40,6 +40,8 @@ namespace fn2
     // compiling, 1 loaded, 2 failed, 3 too long to specialise.
     int JitVariantState( const DeviceProgram* p, int variant );
 
+    // Whether the program's specialised kernel walks grid requests in bricks
+    bool JitWalksBricks( const DeviceProgram& p );
     // Whether the program holds a fused fractal (the unroll variants differ)
     bool JitHasFusedFractal( const DeviceProgram& p );
     // Whether the shared far-cell walk variant differs from the default: a 3D
