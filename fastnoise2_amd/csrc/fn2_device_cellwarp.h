@@ -15,13 +15,25 @@ namespace fn2d
         else if constexpr( D == 3 ) return hashHB3( seed, c[0], c[1], c[2] );
         else return hashHB4( seed, c[0], c[1], c[2], c[3] );
     }
+    // A value of a cell kept in a vector register, in the specialised kernels.
+    // The statement may not be duplicated across a loop's iterations, which
+    // keeps the interpreter's cell loops rolled: its 256^3 warped cellular grid
+    // took 0.85 ms with it, 0.43 without.
+    FN2D int32_t inCellVector( int32_t v )
+    {
+#if defined( __HIPCC_RTC__ )
+        return inVector( v );
+#else
+        return v;
+#endif
+    }
     // bits 1-10 of b as a number minus 511.5: set into the mantissa of 2^22
     // (whose last bit counts halves), which is subtracted again. Exact, and
     // three full-rate instructions instead of a half-rate conversion and more.
     FN2D float centredField( int32_t b )
     {
 #if defined( __HIP_DEVICE_COMPILE__ )
-        const int32_t mask = inVector( 0x7fe ), one = inVector( 0x4a800000 );
+        const int32_t mask = inCellVector( 0x7fe ), one = inCellVector( 0x4a800000 );
         return ibits( (int32_t)__builtin_amdgcn_bitop3_b32( (uint32_t)b, (uint32_t)mask, (uint32_t)one, 0xea ) ) - ( 4194304.0f + 511.5f );
 #else
         return ibits( ( b & 0x7fe ) | 0x4a800000 ) - ( 4194304.0f + 511.5f );
@@ -37,7 +49,7 @@ namespace fn2d
         }
         else if constexpr( D == 3 )
         {
-            h = inVector( h );   // else h + h becomes a second multiplication
+            h = inCellVector( h );   // else h + h becomes a second multiplication
             v[0] = centredField( iadd( h, h ) );
             v[1] = centredField( isrl( h, 10 ) );
             v[2] = centredField( isrl( h, 21 ) );
@@ -299,6 +311,8 @@ namespace fn2d
             // above +inf: unsigned min / max give the results of the float
             // min / max steps above (a NaN distance never displaces a slot, and
             // no slot becomes NaN), without canonicalising their operands.
+            // One median (4.3 cycles) keeps a slot where a minimum and a
+            // maximum (4.3 each) did.
             const uint32_t nb = (uint32_t)fbits( nd );
             if constexpr( SLOTS > 3 ) key[3] = umed3( key[2], key[3], nb );
             if constexpr( SLOTS > 2 ) key[2] = umed3( key[1], key[2], nb );
@@ -342,7 +356,11 @@ namespace fn2d
     // lane's walk, or, in 3D where the c take at most two values per axis (most
     // grid bricks), one of 4 cells a side, which the 64 lanes fill in one
     // round instead of two. Else returns false, having written nothing. HASH:
-    // also keep each cell's hash (CellularValue returns it).
+    // also keep each cell's hash (CellularValue returns it). Warped cellular
+    // 256^3, us per call: 209 with only the box of 5 and the selects and full
+    // roots of before, 188 with this one, umed3, centredField and invSqrtCell
+    // (16.8 M positions, which use no table: 298 and 276). Bound by the vector
+    // ALU's issue; HBM would allow 10.
     template<int D, bool HASH>
     __device__ __forceinline__ bool fillCellTable( const CellParams& cp, const float* pos, int32_t* c, int32_t* origin )
     {

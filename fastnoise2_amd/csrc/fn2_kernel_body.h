@@ -400,8 +400,10 @@ namespace fn2k
         const uint32_t waves = gridDim.x * kWaves;
         // this wave's part of the items beyond the first round: [first, end)
         const fn2::QueuePart q = fn2::queuePart( g, waves, items );
-        const uint32_t first = q.first, end = q.end;
-        uint32_t* myCounter = counter + q.part * fn2::kQueueCounterStride;
+        // said to be the wave's own: else the loop's branches and addresses are
+        // taken for the lanes', and each of 64 lanes issues the atomics below
+        const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane( (int)q.first ), end = (uint32_t)__builtin_amdgcn_readfirstlane( (int)q.end );
+        uint32_t* myCounter = counter + (uint32_t)__builtin_amdgcn_readfirstlane( (int)q.part ) * fn2::kQueueCounterStride;
         for( uint32_t w = g; w < items; )
         {
             const uint32_t t = w / kWaves;
