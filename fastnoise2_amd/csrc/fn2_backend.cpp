@@ -109,6 +109,9 @@ namespace fn2
     bool HipOk( hipError_t e, const char* what )
     {
         if( e == hipSuccess ) return true;
+        // reported here, and not again by the thread's next kernel launch,
+        // whose launcher asks for the last error
+        (void)hipGetLastError();
         SetError( std::string( what ) + ": " + hipGetErrorString( e ) );
         return false;
     }

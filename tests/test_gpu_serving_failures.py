@@ -1,0 +1,54 @@
+"""Serving requests that fail: a destination that its allocation cuts short is
+refused by the copy into it, and the engine and its other requests go on."""
+import numpy as np
+import pytest
+
+import fastnoise2_amd as fn
+from fastnoise2_amd import workloads as W
+from fastnoise2_amd.serve import ServeEngine, SERVE_PLAIN, SERVE_BATCHED, SERVE_GRAPH, SERVE_PERSISTENT
+from conftest import assert_bitexact
+
+pytestmark = pytest.mark.gpu
+
+MODES = [SERVE_BATCHED, SERVE_GRAPH, SERVE_PLAIN, SERVE_PERSISTENT]
+
+
+class Slice:
+    """`count` floats from float `at` of a DeviceArray or PinnedArray (or of what follows it)."""
+
+    def __init__(self, whole, at, count):
+        self.count, self.ptr = count, whole.ptr + 4 * at
+
+
+def engine(mode, capacity=1 << 16):
+    eng = ServeEngine(hbm_budget_bytes=1 << 30, max_batch_points=capacity, mode=mode)
+    return eng, eng.add_tree(W.fbm_simplex_2d().encode())
+
+
+def spec(n):
+    return fn.grid_spec(2, [3.0, -7.0], [n, 1], seed=2)
+
+
+def alone(n):
+    return fn.Node.from_encoded(W.fbm_simplex_2d().encode()).gen_uniform_grid_2d(3.0, -7.0, n, 1, seed=2)
+
+
+@pytest.mark.parametrize("jit", [fn.JIT_OFF, fn.JIT_SYNC])
+@pytest.mark.parametrize("mode", MODES)
+def test_a_failed_request_does_not_fail_the_next(gpu, mode, jit):
+    # a few floats too many, which still lie on the allocation's last page
+    old = fn.set_jit_mode(jit)
+    try:
+        eng, tid = engine(mode)
+        pinned = fn.PinnedArray(1000)
+        want, mm = alone(1000)
+        for at, n in ((0, 1001), (990, 11)):
+            rid = eng.submit(tid, spec(n), out=Slice(pinned, at, n))
+            with pytest.raises(RuntimeError):
+                eng.wait(rid)
+            got, got_mm, _ = eng.wait(eng.submit(tid, spec(1000)))
+            assert_bitexact(got, want, "after the refusal")
+            assert got_mm == mm
+        eng.close()
+    finally:
+        fn.set_jit_mode(old)
