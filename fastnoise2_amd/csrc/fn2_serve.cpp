@@ -118,8 +118,8 @@ namespace
         // where the values go: through the slot's pinned staging buffer (pageable
         // caller memory), straight from the arena into pinned caller memory,
         // or into caller device memory: written there by the batch's kernels
-        // (kDirect, memory of the engine's own device), else by a
-        // device-to-device copy
+        // (kDirect, memory of the engine's own device that WritableInPlace
+        // finds large enough), else by a device-to-device copy
         enum Dest { kStaged, kPinned, kDirect, kDevice } dest = kStaged;
         // results
         bool done = false;
@@ -335,20 +335,20 @@ namespace
             r->tree = treeId;
             r->spec = spec;
             r->hostOut = hostOut;
-            {
-                hipPointerAttribute_t attr;
-                if( hipPointerGetAttributes( &attr, hostOut ) == hipSuccess )
-                    r->dest = attr.type == hipMemoryTypeHost     ? Request::kPinned
-                              : attr.type != hipMemoryTypeDevice ? Request::kStaged
-                              : attr.device == device            ? Request::kDirect
-                                                                 : Request::kDevice;
-                else (void)hipGetLastError();
-            }
             std::string err;
             if( !fn2::FillSpecArgs( spec, r->args, r->points, err ) )
             {
                 fn2::SetError( err );
                 return -1;
+            }
+            {
+                hipPointerAttribute_t attr;
+                if( hipPointerGetAttributes( &attr, hostOut ) == hipSuccess )
+                    r->dest = attr.type == hipMemoryTypeHost                                   ? Request::kPinned
+                              : attr.type != hipMemoryTypeDevice                               ? Request::kStaged
+                              : attr.device == device && WritableInPlace( hostOut, r->points ) ? Request::kDirect
+                                                                                               : Request::kDevice;
+                else (void)hipGetLastError();
             }
             const fn2::DeviceProgram* prog = nullptr;
             {
@@ -779,6 +779,23 @@ namespace
         static int64_t KernelKey( const fn2::DeviceProgram* p, const fn2::JitKernel* k )
         {
             return k ? (int64_t)(uintptr_t)k : p->dimMask * 16 + p->featMask;
+        }
+
+        // Whether the batch's kernels may write a device destination themselves:
+        // its floats are aligned and lie inside one allocation. For any other
+        // the copy decides, which the runtime refuses where the allocation
+        // is too short; a kernel would write past its end.
+        static bool WritableInPlace( const float* out, int64_t points )
+        {
+            hipDeviceptr_t base = nullptr;
+            size_t bytes = 0;
+            if( hipMemGetAddressRange( &base, &bytes, (hipDeviceptr_t)const_cast<float*>( out ) ) != hipSuccess )
+            {
+                (void)hipGetLastError();
+                return false;
+            }
+            const uintptr_t at = (uintptr_t)out - (uintptr_t)base;
+            return (uintptr_t)out % sizeof( float ) == 0 && at <= bytes && (size_t)points <= ( bytes - at ) / sizeof( float );
         }
 
         bool Launch( Slot& s )

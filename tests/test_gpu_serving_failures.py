@@ -52,3 +52,21 @@ def test_a_failed_request_does_not_fail_the_next(gpu, mode, jit):
         eng.close()
     finally:
         fn.set_jit_mode(old)
+
+
+@pytest.mark.parametrize("mode", MODES)
+def test_device_destinations_beyond_their_allocation_are_refused(gpu, mode):
+    # the batch's kernels write device destinations themselves, these not
+    eng, tid = engine(mode)
+    whole = fn.DeviceArray.from_host(np.full(1000, -777.0, np.float32))
+    for at, n in ((0, 1001), (990, 11), (999, 2)):
+        rid = eng.submit(tid, spec(n), out=Slice(whole, at, n))
+        with pytest.raises(RuntimeError):
+            eng.wait(rid)
+        assert (whole.to_host() == -777.0).all()
+    # up to the allocation's last float
+    got_mm = eng.wait(eng.submit(tid, spec(1000), out=Slice(whole, 0, 1000)))[1]
+    want, mm = alone(1000)
+    assert_bitexact(whole.to_host(), want, "after the refusals")
+    assert got_mm == mm
+    eng.close()
