@@ -1087,6 +1087,10 @@ namespace
                 }
                 int si = code >= 0 ? code : -1 - code;
                 Slot& s = slots[si];
+                // A batch that failed part way has launches and copies on its
+                // stream: its requests may not be done, and its tables not
+                // filled anew, before those have ended
+                if( code < 0 ) (void)fn2::HipOk( hipStreamSynchronize( s.stream ), "failed serve batch" );
                 bool ok = code >= 0 && fn2::HipOk( hipEventSynchronize( s.done ), "serve batch" );
                 if( ok )
                 {

@@ -70,3 +70,25 @@ def test_device_destinations_beyond_their_allocation_are_refused(gpu, mode):
     assert_bitexact(whole.to_host(), want, "after the refusals")
     assert got_mm == mm
     eng.close()
+
+
+def test_a_failed_batch_has_ended_when_its_requests_return(gpu):
+    # full batches keep the slots busy while a large request into device
+    # memory and one that is refused queue up behind them: they share a batch
+    n = 1 << 22
+    enc = W.serving_tree().encode()
+    eng = ServeEngine(hbm_budget_bytes=1 << 30, max_batch_points=n, mode=SERVE_BATCHED)
+    tid = eng.add_tree(enc)
+    want, _ = fn.Node.from_encoded(enc).gen_uniform_grid_2d(3.0, -7.0, n // 2, 1, seed=2)
+    whole, short = fn.DeviceArray.from_host(np.zeros(n // 2, np.float32)), fn.PinnedArray(1000)
+    busy = [fn.DeviceArray(n) for _ in range(12)]
+    eng.wait(eng.submit(tid, spec(n), out=busy[0]))   # tunes the tree
+    first = [eng.submit(tid, spec(n), out=b) for b in busy]
+    good, bad = eng.submit(tid, spec(n // 2), out=whole), eng.submit(tid, spec(1001), out=Slice(short, 0, 1001))
+    for rid in (good, bad):
+        with pytest.raises(RuntimeError):
+            eng.wait(rid)
+    assert_bitexact(whole.to_host(), want, "the batch's other request")
+    for rid in first:
+        eng.wait(rid)
+    eng.close()
