@@ -1328,7 +1328,12 @@ FASTNOISE_API int fn2ServeReplay( void* engine, int count, const int* treeIds, c
         int slot = freeSlots.back();
         freeSlots.pop_back();
         int64_t id = e->Submit( treeIds[i], specs[i], pool[slot] );
-        if( id < 0 ) return 1;
+        if( id < 0 )
+        {
+            // the requests submitted so far still write into the pool
+            status = 1;
+            break;
+        }
         pending.emplace_back( id, slot );
         reqIndex.push_back( i );
     }

@@ -92,3 +92,14 @@ def test_a_failed_batch_has_ended_when_its_requests_return(gpu):
     for rid in first:
         eng.wait(rid)
     eng.close()
+
+
+@pytest.mark.parametrize("device_outputs", [False, True])
+def test_a_replay_that_stops_waits_for_what_it_submitted(gpu, device_outputs):
+    # its output buffers are freed when it returns
+    eng, tid = engine(SERVE_BATCHED)
+    specs = [spec(1 << 16)] * 40
+    with pytest.raises(RuntimeError, match="unknown tree id"):
+        eng.replay([tid] * 39 + [tid + 1], specs, None, 64, device_outputs=device_outputs)
+    assert eng.stats()["completed"] == 39
+    eng.close()
