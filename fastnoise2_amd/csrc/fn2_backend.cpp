@@ -993,18 +993,16 @@ FASTNOISE_API int fn2BenchGenerate( const void* node, const fn2GenSpec* spec, fl
     a.nIns = (int32_t)dp->ins.size();
     a.resultReg = dp->resultReg;
     a.out = dOut;
-    // the range is part of the launch, its reduction is not
-    a.minmax = c->dKeys;
     for( int i = 0; i < warmup; i++ )
     {
-        if( !HipOk( LaunchProgram( a, dp, c->stream ), "launch" ) ) return 1;
+        if( !c->LaunchRanged( a, dp, c->stream ) ) return 1;
     }
     if( !HipOk( hipStreamSynchronize( c->stream ), "warmup" ) ) return 1;
     auto t0 = std::chrono::steady_clock::now();
     if( !HipOk( hipEventRecord( c->ev0, c->stream ), "event" ) ) return 1;
     for( int i = 0; i < iters; i++ )
     {
-        if( !HipOk( LaunchProgram( a, dp, c->stream ), "launch" ) ) return 1;
+        if( !c->LaunchRanged( a, dp, c->stream ) ) return 1;
     }
     if( !HipOk( hipEventRecord( c->ev1, c->stream ), "event" ) ) return 1;
     if( !HipOk( hipStreamSynchronize( c->stream ), "timed launches" ) ) return 1;

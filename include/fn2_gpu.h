@@ -71,8 +71,9 @@ FASTNOISE_API int fn2GenerateDeviceNoAlloc( const void* node, const fn2GenSpec* 
 FASTNOISE_API size_t fn2NoAllocScratchBytes( void );
 
 /* Times `iters` back-to-back generator launches (each writes all points of
- * `spec` to dOut and folds them into the call's min/max) after `warmup`
- * launches, with HIP events on the launch stream. msPerLaunch: average event
+ * `spec` to dOut and folds them into the call's min/max, with the reduction
+ * launch that this takes beyond 512 blocks) after `warmup` launches, with HIP
+ * events on the launch stream. msPerLaunch: average event
  * time per launch; wallMsPerLaunch: host wall time per launch from the first
  * launch to the completion of the last. */
 FASTNOISE_API int fn2BenchGenerate( const void* node, const fn2GenSpec* spec, float* dOut, int warmup, int iters, double* msPerLaunch, double* wallMsPerLaunch );

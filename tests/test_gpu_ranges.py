@@ -31,3 +31,17 @@ def test_range_is_that_of_the_values(gpu, n, jit):
             assert node.generate_device(fn.positions_spec(pos), dev) == mm
     finally:
         fn.set_jit_mode(old)
+
+
+def test_timed_launches_include_the_reduction(gpu):
+    # 512 blocks of 256 points leave their pairs to the host, one more takes a
+    # reduction launch, which costs at least a microsecond
+    old = fn.set_jit_mode(fn.JIT_SYNC)
+    try:
+        node = fn.Node.from_encoded(S("Simplex", feature_scale=30.0).encode())
+        out = fn.DeviceArray(131073)
+        ms = {n: min(node.bench_device(fn.grid_spec(2, [0.0, 0.0], [n, 1]), out, warmup=5, iters=200)[0] for _ in range(5))
+              for n in (131072, 131073)}
+        assert ms[131073] - ms[131072] > 1.0e-3
+    finally:
+        fn.set_jit_mode(old)
