@@ -238,6 +238,19 @@ namespace fn2
         return true;
     }
 
+    int ProgramTables( const std::vector<Ins>& ins )
+    {
+        int t = 0;
+        for( const Ins& in : ins )
+        {
+            const int grad = in.dim == 2 ? kTableGrad2 : in.dim == 3 ? kTableGrad3 : kTableGrad4;
+            const int leaf = in.op == OP_FRACTAL_LEAF ? in.p[0] : in.op;
+            if( leaf == OP_PERLIN || leaf == OP_SIMPLEX || leaf == OP_SUPERSIMPLEX ) t |= grad;
+            if( ( in.op == OP_WARP_SIMPLEX || in.op == OP_WARP_SUPERSIMPLEX ) && in.dim == 3 && in.p[0] != 1 ) t |= kTableOrtho3;
+        }
+        return t;
+    }
+
     static bool SameProgram( const DeviceProgram* d, const Program& p )
     {
         return d->resultReg == p.resultReg && d->dims == p.dims && d->ins.size() == p.ins.size() && d->konst.size() == p.konst.size() &&
@@ -283,6 +296,7 @@ namespace fn2
         d->featMask = p.featMask;
         d->dims = p.dims;
         d->regs = regs;
+        d->tables = ProgramTables( p.ins );
         size_t insBytes = std::max<size_t>( 1, p.ins.size() ) * sizeof( Ins );
         // padded so that a window starting at the last constant stays in bounds
         size_t kBytes = ( p.konst.size() + 16 ) * sizeof( float );
@@ -661,6 +675,7 @@ namespace fn2
         a.ins = dp->dIns;
         a.konst = dp->dKonst;
         a.regs = dp->regs;
+        a.tables = dp->tables;
         a.nIns = (int32_t)dp->ins.size();
         a.resultReg = dp->resultReg;
 
@@ -953,6 +968,7 @@ FASTNOISE_API int fn2GenerateDevice( const void* node, const fn2GenSpec* spec, f
     a.ins = dp->dIns;
     a.konst = dp->dKonst;
     a.regs = dp->regs;
+    a.tables = dp->tables;
     a.nIns = (int32_t)dp->ins.size();
     a.resultReg = dp->resultReg;
     a.out = dOut;
@@ -990,6 +1006,7 @@ FASTNOISE_API int fn2BenchGenerate( const void* node, const fn2GenSpec* spec, fl
     a.ins = dp->dIns;
     a.konst = dp->dKonst;
     a.regs = dp->regs;
+    a.tables = dp->tables;
     a.nIns = (int32_t)dp->ins.size();
     a.resultReg = dp->resultReg;
     a.out = dOut;

@@ -23,6 +23,7 @@ namespace fn2
         int featMask = 0;
         int dims = 0;    // of the starting positions (programs are cached per dimensionality)
         int regs = 1;    // registers used: every operand lies below this
+        int tables = 0;  // LDS tables its kernels read (kTable* bits)
         Ins* dIns = nullptr;
         float* dKonst = nullptr;
         // the specialised-kernel variant single calls run (fn2_jit.h; same
@@ -103,6 +104,8 @@ namespace fn2
     // register operands (regs = the register count it needs) and constant
     // windows; false with `err` set when it is malformed
     bool ValidateProgram( const Program& p, int& regs, std::string& err );
+    // The LDS tables (kTable* bits) a program's instructions read
+    int ProgramTables( const std::vector<Ins>& ins );
     const DeviceProgram* GetDeviceProgram( const Program& p );
     // The cached device program of `p` if one exists, else null (never creates one)
     const DeviceProgram* FindDeviceProgram( const Program& p );

@@ -131,20 +131,6 @@ namespace fn2
             return true;
         }
 
-        // The LDS tables (kTable*) the program's instructions read
-        int Tables( const DeviceProgram& p )
-        {
-            int t = 0;
-            for( const Ins& in : p.ins )
-            {
-                const int grad = in.dim == 2 ? kTableGrad2 : in.dim == 3 ? kTableGrad3 : kTableGrad4;
-                const int leaf = in.op == OP_FRACTAL_LEAF ? in.p[0] : in.op;
-                if( leaf == OP_PERLIN || leaf == OP_SIMPLEX || leaf == OP_SUPERSIMPLEX ) t |= grad;
-                if( ( in.op == OP_WARP_SIMPLEX || in.op == OP_WARP_SUPERSIMPLEX ) && in.dim == 3 && in.p[0] != 1 ) t |= kTableOrtho3;
-            }
-            return t;
-        }
-
         // Each instruction becomes an `execIns` instantiated for its own op,
         // dimensionality and (fused fractal) leaf op, so the compiler sees only
         // the code that instruction runs.
@@ -168,7 +154,7 @@ namespace fn2
                  "static constexpr int kDims = " << p.dims << ";\n"
                  "static constexpr bool kBricks = " << ( PrunedCellular( p ) ? "true" : "false" ) << ";\n"
                  "static constexpr bool kWide = " << ( Wide( p ) ? "true" : "false" ) << ";\n"
-                 "static constexpr int kTables = " << Tables( p ) << ";\n"
+                 "static constexpr int kTables = " << ProgramTables( p.ins ) << ";\n"
                  "__device__ __forceinline__ float operator()( const fn2::GenArgs& a, float* R ) const {\n";
             // long programs get a register fence between instructions: measured
             // on MI355X, a 355-instruction tree needs 256 VGPRs without (one wave

@@ -94,6 +94,7 @@ namespace fn2
         const float* pos[4];     // position arrays (device); tileable: cos x, cos y, sin x, sin y tables
         int32_t ppt;             // batched kernel: points per lane of each block of this job
         int32_t regs;            // registers the program uses (the interpreter's file holds as many)
+        int32_t tables;          // LDS tables the program reads (kTable* bits)
         int32_t rangeStride;     // ints between the slots of the range record (kRangePerBlock: its pairs)
         int32_t rangeSlots;      // slots of the range record (a power of two), or kRangePerBlock
         // index of this job's first point in its request: a request split

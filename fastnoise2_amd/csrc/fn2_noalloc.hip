@@ -178,6 +178,7 @@ FASTNOISE_API int fn2GenerateDeviceNoAlloc( const void* node, const fn2GenSpec* 
     a.ins = dIns;
     a.konst = dKonst;
     a.regs = regs;
+    a.tables = ProgramTables( p.ins );
     a.nIns = (int32_t)p.ins.size();
     a.resultReg = p.resultReg;
     a.out = dOut;

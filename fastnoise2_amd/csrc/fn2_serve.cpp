@@ -445,6 +445,7 @@ namespace
             r->args.ins = prog->dIns;
             r->args.konst = prog->dKonst;
             r->args.regs = prog->regs;
+            r->args.tables = prog->tables;
             r->args.nIns = (int32_t)prog->ins.size();
             r->args.resultReg = prog->resultReg;
             r->tSubmit = Clock::now();
@@ -674,6 +675,7 @@ namespace
             a.ins = prog->dIns;
             a.konst = prog->dKonst;
             a.regs = prog->regs;
+            a.tables = prog->tables;
             a.nIns = (int32_t)prog->ins.size();
             a.resultReg = prog->resultReg;
             a.out = tuneOut;
