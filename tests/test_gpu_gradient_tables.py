@@ -1,8 +1,9 @@
 """The LDS tables behind gradient selection and the orthogonal warp matrices
 against the oracle, bit for bit: every leaf alone and fused into fractals, and
 the simplex-type warps, in 2D, 3D and 4D, on the interpreter, on specialised
-kernels and in serving batches of the smallest blocks, over enough points to
-read every entry, with steps of either sign and huge and non-finite offsets."""
+kernels and in serving batches that mix programs with different tables, over
+enough points to read every entry, with steps of either sign and huge and
+non-finite offsets."""
 import numpy as np
 import pytest
 
@@ -56,9 +57,10 @@ def test_grids_match_oracle(jit, name, dims):
 
 @pytest.mark.parametrize("mode", [SERVE_BATCHED, SERVE_PERSISTENT])
 def test_batches_match_oracle(jit, mode):
-    # tiles of 64, 128 and 256 threads fill the tables alike
+    # the blocks of a batch fill the tables of their own job's program (the
+    # work queue's those of its kernel)
     eng = ServeEngine(hbm_budget_bytes=1 << 30, max_batch_points=1 << 18, mode=mode)
-    names = ["Perlin", "FBm Simplex", "DomainWarpSimplex Orthogonal Gradient Matrix"]
+    names = ["Value", "Perlin", "FBm Simplex", "DomainWarpSimplex Gradient Outer Product", "DomainWarpSimplex Orthogonal Gradient Matrix"]
     ids = {}
     for n in names:
         t = eng.add_tree(TREES[n].encode())
