@@ -84,10 +84,12 @@ namespace fn2d
     // arguments with normal results, built from the hardware estimates
     // (v_sqrt_f32 / v_rcp_f32, both within 1 ulp) plus fma corrections,
     // without the zero / denormal / infinity scaling of the general IEEE
-    // routines. Used where the argument range is known: the cellular jitter
-    // vector's squared length, which lies in [0.5, 2.2e6] because every
-    // component is a half-integer. fn2SelfTestMath checks them against the
-    // IEEE results over whole binades.
+    // routines. Used where the argument range is known or tested: the squared
+    // length of a 2D cellular jitter vector, which lies in [0.5, 2.2e6]
+    // because every component is a half-integer, and the distances that
+    // CellularDistance returns, where invSqrtPosHolds (2^-60 to 2^61).
+    // fn2SelfTestMath checks them against the IEEE results over whole
+    // binades of both ranges.
 #if defined( __HIP_DEVICE_COMPILE__ )
     FN2D float sqrtPosRN( float x )
     {
@@ -109,21 +111,9 @@ namespace fn2d
         return __builtin_fmaf( e, y, y );
     }
 
-    // sqrtPosRN for arguments on which the hardware estimate is never above
-    // the correctly rounded root, so only the step up needs testing: the
-    // squared lengths of 3D and 4D cellular jitter vectors (N / 4 for a sum N
-    // of three or four odd squares below 2^22), checked exhaustively on the
-    // device by the math tests
-    FN2D float sqrtPosRNFromBelow( float x )
-    {
-        const float s = __builtin_amdgcn_sqrtf( x );
-        const float up = ibits( fbits( s ) + 1 );
-        return __builtin_fmaf( -up, s, x ) > 0.0f ? up : s;
-    }
 #else
     FN2D float sqrtPosRN( float x ) { return __builtin_sqrtf( x ); }
     FN2D float recipPosRN( float b ) { return 1.0f / b; }
-    FN2D float sqrtPosRNFromBelow( float x ) { return __builtin_sqrtf( x ); }
 #endif
     // Square root for bounds that carry margins far above 1 ulp (the
     // cellular walks' pruning limits): on the device the hardware estimate
@@ -142,8 +132,11 @@ namespace fn2d
     // Selects as arithmetic on vector registers. A compare and a select on a
     // scalar mask issue at half the rate of the rest (see gradDot3's tables),
     // so where a < b decides several selects, the sign of a - b is spread over
-    // a mask once. a - b is negative exactly where a < b (denormals are kept);
-    // a NaN may go either way, and its results are NaN on both.
+    // a mask once. a - b is negative exactly where a < b (denormals are kept)
+    // unless a is -0 and b is +0, which gives -0 and a set mask: only for
+    // values that are never -0, as the callers' are (fractions x - floor( x ),
+    // whose zeros are +0, and sums with one). A NaN may go either way, and its
+    // results are NaN on both. negativeMask, signBit: the same of one value.
     FN2D int32_t lessMask( float a, float b ) { return fbits( a - b ) >> 31; }
     FN2D int32_t negativeMask( float a ) { return fbits( a ) >> 31; }
     FN2D int32_t signBit( float a ) { return fbits( a ) & (int32_t)0x80000000u; }
@@ -159,14 +152,15 @@ namespace fn2d
     FN2D float bitSelect( int32_t mask, float a, float b ) { return ibits( bitSelect( mask, fbits( a ), fbits( b ) ) ); }
     // 1.0f where the mask is set, else 0
     FN2D float maskedOne( int32_t mask ) { return ibits( mask & 0x3f800000 ); }
-    // max( a, 0 ) of a value known to lie below 1 (or NaN, which gives 0):
-    // folds into the instruction that makes a as its clamp modifier
+    // a limited to [0, 1] (NaN gives 0), for max( a, 0 ) of a value known to
+    // lie below 1, as the falloffs do (0.7 at most): folds into the
+    // instruction that makes a as its clamp modifier
     FN2D float clampPositive( float a )
     {
 #if defined( __HIP_DEVICE_COMPILE__ )
         return __builtin_amdgcn_fmed3f( a, 0.0f, 1.0f );
 #else
-        return a > 0.0f ? a : 0.0f;
+        return a > 0.0f ? ( a < 1.0f ? a : 1.0f ) : 0.0f;
 #endif
     }
     // the same value in a vector register: instructions with an operand in a

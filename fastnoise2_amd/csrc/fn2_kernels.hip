@@ -61,6 +61,16 @@ __global__ void __launch_bounds__( BLOCK ) fn2_generate_queue( const fn2::GenArg
     fn2k::generateQueue<BLOCK>( jobs, tileJob, tileBase, nTiles, counter, Interpreted<DM, FT>() );
 }
 
+// Self-test op 5: the square root by the hardware estimate and a correction
+// upward only. No node takes it any more (invSqrtCell replaced it); it stays
+// for callers of the self-test.
+__device__ __forceinline__ float sqrtFromBelow( float x )
+{
+    const float s = __builtin_amdgcn_sqrtf( x );
+    const float up = ibits( fbits( s ) + 1 );
+    return __builtin_fmaf( -up, s, x ) > 0.0f ? up : s;
+}
+
 __global__ void fn2_selftest_math( int op, const float* in, float* out, int n )
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -68,7 +78,7 @@ __global__ void fn2_selftest_math( int op, const float* in, float* out, int n )
     {
         float x = in[i];
         out[i] = op == 0 ? sqrtPosRN( x ) : op == 1 ? recipPosRN( x ) : op == 2 ? invSqrtPos( x ) : op == 3 ? invSqrt( x )
-               : op == 4 ? __builtin_amdgcn_sqrtf( x ) : op == 5 ? sqrtPosRNFromBelow( x ) : invSqrtCell<3>( x );
+               : op == 4 ? __builtin_amdgcn_sqrtf( x ) : op == 5 ? sqrtFromBelow( x ) : invSqrtCell<3>( x );
     }
 }
 

@@ -1,5 +1,5 @@
 """Exhaustive check of the fast correctly rounded sqrt / reciprocal that the
-cellular nodes use for the jitter vector length: every float of every binade
+cellular nodes use for the 2D jitter vector length: every float of every binade
 the argument can take, against the IEEE results (numpy float32 sqrt and
 division are correctly rounded)."""
 import numpy as np
@@ -61,9 +61,9 @@ def cell_lengths(dims):
 
 @pytest.mark.parametrize("dims", [3, 4])
 def test_upward_corrected_sqrt_exact_on_cell_lengths(gpu, dims):
-    # the 3D / 4D cellular nodes correct the hardware square root estimate
-    # upward only; on every argument they can pass that must be the
-    # correctly rounded root
+    # on the squared lengths of 3D / 4D jitter vectors the hardware square
+    # root estimate, corrected upward only, must be the correctly rounded root
+    # (the nodes' own reciprocal root of them: test_gpu_cell_math.py)
     x = cell_lengths(dims)
     assert np.array_equal(x.astype(np.float64) * 4, np.arange(dims, dims * {3: 1023, 4: 255}[dims] ** 2 + 1, 8))
     din = fn.DeviceArray(x.size)
