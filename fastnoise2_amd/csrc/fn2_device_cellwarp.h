@@ -18,7 +18,7 @@ namespace fn2d
     // A value of a cell kept in a vector register, in the specialised kernels.
     // The statement may not be duplicated across a loop's iterations, which
     // keeps the interpreter's cell loops rolled: its 256^3 warped cellular grid
-    // took 0.85 ms with it, 0.43 without.
+    // took 0.85 ms with it, 0.40 without.
     FN2D int32_t inCellVector( int32_t v )
     {
 #if defined( __HIPCC_RTC__ )

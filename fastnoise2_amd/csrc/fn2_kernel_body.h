@@ -187,11 +187,13 @@ namespace fn2k
     // by the writes: with a point per lane these kernels spent about 100
     // cycles of a SIMD per wave and point, most of it on the index, which was
     // as long as the writes took. One point per lane -> four on MI355X, GB/s
-    // in turn into several buffers: checkerboard 4096^2 3921 -> 5366, 8192^2
-    // 4385 -> 6600, 16384^2 5327 -> 6944; white noise 8192^2 3790 -> 6376; a
-    // constant 8192^2 4890 -> 6180 (a fill of 256 MB: 6700). The output has to
-    // lie on 16 bytes; programs with more to do per point gain nothing and
-    // would need four points' registers.
+    // without a range, in turn into several buffers: checkerboard 4096^2 3921
+    // -> 5250, 8192^2 4385 -> 6010, 16384^2 5327 -> 6210; white noise 8192^2
+    // 3790 -> 6376; a constant 8192^2 4890 -> 6180 (a fill of 256 MB: 6700).
+    // With a range, in longer runs (WideGridFor): whole calls of 8192^2 into
+    // one buffer 74 -> 57 us, but the kernel of 16384^2 5537 -> 5502 GB/s. The
+    // output has to lie on 16 bytes; programs with more to do per point gain
+    // nothing and would need four points' registers.
     // RANGED: the call wants its range (a copy without it saves a fifth of
     // the instructions).
     template<int BLOCK, bool RANGED, class Prog>
@@ -224,7 +226,8 @@ namespace fn2k
                 v[k] = prog( a, fresh.R );
                 if constexpr( RANGED ) widen( v[k], mn, mx );
             }
-            // a plain store: streaming ones were slower (WideGridFor's figures)
+            // a plain store: with streaming ones, and the blocks striding by
+            // the grid, checkerboard 8192^2 took 58 us instead of 48
             *reinterpret_cast<Vec4*>( a.out + 4 * g ) = v;
         }
         const uint32_t rest = 4 * groups + threadIdx.x;

@@ -225,14 +225,25 @@ namespace
 
     // Blocks of a single-call kernel of a cheap program, which writes four
     // points per lane and round (4 KiB a block) and takes a contiguous run of
-    // rounds per block (fn2k::generateWide): 4096 blocks or runs of four
-    // rounds, and of two beyond 64 MB, where short runs keep the blocks at
-    // work at one time writing close together. Measured on MI355X, GB/s of
-    // checkerboards of 64 MB / 256 MB / 1 GB in turn into several buffers: one
-    // point per lane 3921 / 4385 / 5327; 4096 blocks 5356 / 5696 / 5570, 16384
-    // 4696 / 6031 / 5378, 32768 4680 / 6532 / 5468, 65536 4670 / 5700 / 5883 (a
-    // fill of 256 MB: 6715). With a range every block costs a pair to reduce:
-    // at most 8192.
+    // rounds per block (fn2k::generateWide): at least 4096 blocks where there
+    // are as many rounds, runs of four rounds at most up to 16,384 rounds (64
+    // MiB), runs of two beyond, where short runs keep the blocks at work at one
+    // time writing close together. Checkerboards without a range on MI355X,
+    // GB/s in turn into several buffers, by their runs (the rule's in brackets):
+    //
+    //     MB        17    34    67    81   100   134   169   213   268   537  1074
+    //     run 1   2649  3658  4917  5209  5479  5886  6198  6388  6572  6853  7071
+    //     run 2   2632  3889  5263 (5447 5611  5807  5843  5935  6021  6159  6217)
+    //     run 4  (2594  3890  5269) 5325  5383  5669  5530  5500  5803  5730  5840
+    //     run 8   2637  3940  5247  5096  5254  5308  5260  5306  5461  5335  5486
+    //
+    // One point per lane reached 3921 at 67 MB, 4385 at 268 and 5327 at 1074.
+    // Runs of one are faster still above 110 MB and slower below.
+    // With a range every block costs a pair to reduce, so there are at most
+    // 8192 blocks, and beyond 64 MiB their runs grow with the image: 32 rounds
+    // at 1074 MB. Whole calls with their range, GB/s, 67 / 134 / 268 / 1074 MB:
+    // 2215 / 3239 / 3993 / 5017, with up to 16,384 blocks in runs of two 2023 /
+    // 2901 / 4423 / 4785.
     unsigned WideGridFor( int64_t total, bool ranged )
     {
         const int64_t rounds = std::max<int64_t>( 1, ( total / 4 + kBlock - 1 ) / kBlock );

@@ -177,8 +177,13 @@ FASTNOISE_API int fn2ServeAddTree( void* engine, const char* encodedTree );
 /* Submits a request: tree id, generation spec (grid or tileable; host
  * positions are not accepted), output buffer of the spec's point count.
  * The output may be pageable host memory (staged through pinned memory),
- * pinned host memory (filled straight from the device) or device memory
- * (a device-to-device copy). A request larger than one batch
+ * pinned host memory (filled straight from the device) or device memory: of
+ * the engine's own device, the batch's kernels write it in place, so parts of
+ * it change at any time between this call and the request's completion;
+ * requests in flight at one time must not share any of it. Memory of another
+ * device is filled by a copy, and so is a destination that does not lie whole
+ * inside one allocation, which the copy refuses: the request fails, and with
+ * it the others of its batch. A request larger than one batch
  * (maxBatchPoints) runs as several parts in successive batches and completes
  * when the last part has. Returns a request id (>= 0) or -1 on bad arguments.
  * The call does not block on the GPU. */
