@@ -74,24 +74,39 @@ def test_device_destinations_beyond_their_allocation_are_refused(gpu, mode):
 
 def test_a_failed_batch_has_ended_when_its_requests_return(gpu):
     # full batches keep the slots busy while a large request into device
-    # memory and one that is refused queue up behind them: they share a batch
+    # memory and one that is refused queue up behind them and share a batch
+    # (tried again should the dispatcher have taken the first alone)
     n = 1 << 22
+    grid = [fn.grid_spec(3, [3.0, -7.0, 1.0], [128, 128, z], seed=2) for z in (n >> 14, n >> 15)]
     enc = W.serving_tree().encode()
-    eng = ServeEngine(hbm_budget_bytes=1 << 30, max_batch_points=n, mode=SERVE_BATCHED)
-    tid = eng.add_tree(enc)
-    want, _ = fn.Node.from_encoded(enc).gen_uniform_grid_2d(3.0, -7.0, n // 2, 1, seed=2)
-    whole, short = fn.DeviceArray.from_host(np.zeros(n // 2, np.float32)), fn.PinnedArray(1000)
-    busy = [fn.DeviceArray(n) for _ in range(12)]
-    eng.wait(eng.submit(tid, spec(n), out=busy[0]))   # tunes the tree
-    first = [eng.submit(tid, spec(n), out=b) for b in busy]
-    good, bad = eng.submit(tid, spec(n // 2), out=whole), eng.submit(tid, spec(1001), out=Slice(short, 0, 1001))
-    for rid in (good, bad):
-        with pytest.raises(RuntimeError):
-            eng.wait(rid)
-    assert_bitexact(whole.to_host(), want, "the batch's other request")
-    for rid in first:
-        eng.wait(rid)
-    eng.close()
+    old = fn.set_jit_mode(fn.JIT_OFF)
+    try:
+        eng = ServeEngine(hbm_budget_bytes=1 << 30, max_batch_points=n, mode=SERVE_BATCHED)
+        tid = eng.add_tree(enc)
+        want, _ = fn.Node.from_encoded(enc).gen_uniform_grid_3d(3.0, -7.0, 1.0, 128, 128, n >> 15, seed=2)
+        short, busy = fn.PinnedArray(1000), [fn.DeviceArray(n) for _ in range(12)]
+        eng.wait(eng.submit(tid, grid[0], out=busy[0]))   # tunes the tree
+        eng.wait(eng.submit(tid, spec(1000)))
+        for _ in range(5):
+            whole = fn.DeviceArray.from_host(np.zeros(n // 2, np.float32))
+            first = [eng.submit(tid, grid[0], out=b) for b in busy]
+            good, bad = eng.submit(tid, grid[1], out=whole), eng.submit(tid, spec(1001), out=Slice(short, 0, 1001))
+            with pytest.raises(RuntimeError):
+                eng.wait(bad)
+            got = whole.to_host()
+            try:
+                eng.wait(good)
+            except RuntimeError:
+                break
+            finally:
+                for rid in first:
+                    eng.wait(rid)
+        else:
+            pytest.fail("the two requests never shared a batch")
+        assert_bitexact(got, want, "the batch's other request")
+        eng.close()
+    finally:
+        fn.set_jit_mode(old)
 
 
 @pytest.mark.parametrize("device_outputs", [False, True])
