@@ -959,6 +959,7 @@ FASTNOISE_API int fn2GenerateDevice( const void* node, const fn2GenSpec* spec, f
         if( outputMinMax ) { outputMinMax[0] = FastNoise::kInfinity; outputMinMax[1] = -FastNoise::kInfinity; }
         return 0;
     }
+    if( !dOut ) { SetError( "null output buffer" ); return 1; }
     const DeviceProgram* dp = nullptr;
     if( !CompileForDevice( static_cast<const FastNoise::Generator*>( node ), a.dims, dp, nullptr ) ) return 1;
     CallContext* c = AcquireContext();
@@ -998,6 +999,7 @@ FASTNOISE_API int fn2BenchGenerate( const void* node, const fn2GenSpec* spec, fl
     std::string err;
     if( !EnsureDevice() ) return 1;
     if( !FillSpecArgs( *spec, a, total, err ) ) { SetError( err ); return 1; }
+    if( total > 0 && !dOut ) { SetError( "null output buffer" ); return 1; }
     const DeviceProgram* dp = nullptr;
     if( !CompileForDevice( static_cast<const FastNoise::Generator*>( node ), a.dims, dp, nullptr ) ) return 1;
     CallContext* c = AcquireContext();

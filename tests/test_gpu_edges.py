@@ -206,3 +206,13 @@ def test_fused_simplex_bricks_on_ragged_grids(gpu, kind):
                     assert mm == ref_mm
     finally:
         fn.set_jit_mode(old)
+
+
+@pytest.mark.parametrize("minmax", [True, False])
+def test_null_device_outputs_are_refused(gpu, minmax):
+    node = fn.Node.from_encoded(TREE.encode())
+    spec = fn.grid_spec(2, [0.0, 0.0], [8, 8])
+    for call in (lambda: node.generate_device(spec, None, minmax=minmax), lambda: node.bench_device(spec, None, 1, 1)):
+        with pytest.raises(RuntimeError, match="null output buffer"):
+            call()
+    assert node.generate_device(fn.grid_spec(2, [0.0, 0.0], [0, 8]), None) == (float("inf"), float("-inf"))
